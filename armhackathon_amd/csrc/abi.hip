@@ -136,6 +136,25 @@ ScratchOrder* scratch_order() {
 
 namespace armscan {
 
+// The calling thread's own source of scratch (arm_scan_thread_scratch) and what it has
+// given since it was set. A stream-ordered allocation and its free cost the host 9 us of a
+// call, 14 with the kernels between them, where torch's caching allocator takes 1.
+struct ThreadScratch {
+  static constexpr int kMost = 8;  // a call takes at most three
+  void* (*alloc)(void*, size_t) = nullptr;
+  void* ctx = nullptr;
+  void* given[kMost] = {};
+  int n = 0;
+};
+static thread_local ThreadScratch t_scratch;
+
+void thread_scratch(void* (*alloc)(void*, size_t), void* ctx) {
+  t_scratch.alloc = alloc;
+  t_scratch.ctx = ctx;
+  t_scratch.n = 0;
+}
+
+
 // Per-call scratch (gate records, SS2D planes, segment maps, cos/sin) comes from a
 // memory pool the library owns, one per device, created on first use and kept until
 // the process ends. Its release threshold keeps freed blocks for the next call, so a
@@ -143,6 +162,19 @@ namespace armscan {
 // pool, which the caller or torch may use, keeps its own settings. Where a pool cannot
 // be created, the scratch comes from the default pool as it is.
 hipError_t stream_alloc(void** p, size_t bytes, hipStream_t st) {
+  if (t_scratch.alloc != nullptr && t_scratch.n < ThreadScratch::kMost) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+      (void)hipGetLastError();  // e.g. the null stream beside a capture: the pool, as ever
+      status = hipStreamCaptureStatusActive;
+    }
+    if (status == hipStreamCaptureStatusNone) {
+      *p = t_scratch.alloc(t_scratch.ctx, bytes);
+      if (*p == nullptr) return hipErrorOutOfMemory;
+      t_scratch.given[t_scratch.n++] = *p;
+      return hipSuccess;
+    }
+  }
   constexpr int kMaxDevices = 64;
   static std::atomic<hipMemPool_t> pools[kMaxDevices] = {};
   static std::atomic<bool> no_pool[kMaxDevices] = {};
@@ -179,11 +211,21 @@ hipError_t stream_alloc(void** p, size_t bytes, hipStream_t st) {
   return hipMallocFromPoolAsync(p, bytes, pool, st);
 }
 
+hipError_t stream_free(void* p, hipStream_t st) {
+  for (int i = 0; i < t_scratch.n; ++i)
+    if (t_scratch.given[i] == p) return hipSuccess;  // its owner gives it back
+  return hipFreeAsync(p, st);
+}
+
 }  // namespace armscan
 
 extern "C" {
 
 uint32_t arm_scan_abi_version(void) { return ARM_SCAN_ABI_VERSION; }
+
+void arm_scan_thread_scratch(void* (*alloc)(void* ctx, size_t bytes), void* ctx) {
+  armscan::thread_scratch(alloc, ctx);
+}
 
 const char* arm_scan_last_error(void) { return g_last_error.c_str(); }
 
@@ -423,7 +465,7 @@ static int mamba3_call(const ArmMamba3Dims* dims, const float* q, const float* k
       p.cos = cs;
       p.sin = cs + n_cs;
       if (e == hipSuccess) e = armscan::m3_scan(p, st);
-      const hipError_t ef = hipFreeAsync(cs, st);
+      const hipError_t ef = armscan::stream_free(cs, st);
       return run(e != hipSuccess ? e : ef, "mamba3 (angle pre-pass, then scan) launch");
     }
   }
@@ -677,7 +719,7 @@ int arm_scan_ss2d_f32(const ArmSS2DDims* dims, const float* u, const float* delt
         }
       }
       int rc = e == hipSuccess ? ARM_SCAN_OK : hip_fail(e, "ss2d launch");
-      const hipError_t fe = hipFreeAsync(scratch, st);
+      const hipError_t fe = armscan::stream_free(scratch, st);
       if (rc == ARM_SCAN_OK && fe != hipSuccess) rc = hip_fail(fe, "ss2d scratch free");
       return rc;
     }
@@ -755,7 +797,7 @@ int arm_scan_ss2d_f32(const ArmSS2DDims* dims, const float* u, const float* delt
     }
   } while (false);
   if (e != hipSuccess) rc = hip_fail(e, "ss2d launch");
-  hipError_t fe = hipFreeAsync(scratch, st);
+  hipError_t fe = armscan::stream_free(scratch, st);
   if (rc == ARM_SCAN_OK && fe != hipSuccess) rc = hip_fail(fe, "ss2d scratch free");
   return rc;
 }

@@ -1335,7 +1335,7 @@ hipError_t run_tile(M1Kern& k, bool rev, float* scratch_p, size_t scratch_bytes,
   e = rev ? launch_tile<M1_TILE_I, true, SIO, ALN, DWBC>(k, st)
           : launch_tile<M1_TILE_I, false, SIO, ALN, DWBC>(k, st);
   if (k.segmap && !scratch_p) {
-    const hipError_t fe = hipFreeAsync(k.segmap, st);
+    const hipError_t fe = stream_free(k.segmap, st);
     if (e == hipSuccess) e = fe;
   }
   return e;
@@ -1463,7 +1463,7 @@ hipError_t m1_scan_chunked(const M1Problem& pr, hipStream_t st) {
     k.bpo = off;
     e = run_tile<0, false, false>(k, rev, nullptr, 0, st);
   }
-  const hipError_t fe = hipFreeAsync(pad, st);
+  const hipError_t fe = stream_free(pad, st);
   return e != hipSuccess ? e : fe;
 }
 

@@ -274,7 +274,7 @@ hipError_t m3_angles_to_cos_sin(const float* angles, const float* dt, size_t bat
   hipLaunchKernelGGL(m3_angles_kernel, dim3((unsigned)blocks), dim3(kAngThreads), 0, st, k);
   hipError_t e = hipGetLastError();
   if (k.segs > 1) {
-    const hipError_t ef = hipFreeAsync(k.seg_tot, st);
+    const hipError_t ef = stream_free(k.seg_tot, st);
     if (e == hipSuccess) e = ef;
   }
   return e;

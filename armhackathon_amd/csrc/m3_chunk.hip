@@ -1516,7 +1516,7 @@ hipError_t m3_scan_chunked(const M3Problem& pr, hipStream_t st) {
     const size_t ds = (size_t)k.nsub * k.nseq, ts = k.ang ? ds * 64 : 0;
     e = stream_alloc((void**)&k.fold, (fs + ds + ts) * sizeof(float), st);
     if (e != hipSuccess) {
-      (void)hipFreeAsync(k.rec, st);
+      (void)stream_free(k.rec, st);
       return e;
     }
     k.fold_decay = k.fold + fs;
@@ -1538,9 +1538,9 @@ hipError_t m3_scan_chunked(const M3Problem& pr, hipStream_t st) {
     else if (R == 2) e = launch_chunk_pt<2, true>(k, kf, rev, st);
     else e = launch_chunk_pt<4, true>(k, kf, rev, st);
   }
-  hipError_t fe = hipFreeAsync(k.rec, st);
+  hipError_t fe = stream_free(k.rec, st);
   if (k.fold) {
-    const hipError_t fe2 = hipFreeAsync(k.fold, st);
+    const hipError_t fe2 = stream_free(k.fold, st);
     if (fe == hipSuccess) fe = fe2;
   }
   return e != hipSuccess ? e : fe;

@@ -179,8 +179,10 @@ hipError_t m3_scan_sequential(const M3Problem& p, hipStream_t st);
 bool m3_chunk_supported(const M3Problem& p);
 hipError_t m3_scan_chunked(const M3Problem& p, hipStream_t st);
 
-// Stream-ordered scratch from the device's default pool, whose release threshold
-// is raised once per device so that freed blocks stay cached between calls.
+// Stream-ordered scratch: from the calling thread's own source (arm_scan_thread_scratch)
+// where it set one and st is not being captured, else from the library's pool.
 hipError_t stream_alloc(void** p, size_t bytes, hipStream_t st);
+// Gives it back after what has been enqueued on st.
+hipError_t stream_free(void* p, hipStream_t st);
 
 }  // namespace armscan

@@ -29,7 +29,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _ffi
-from .op import _CALLS, _c, _device_of, _ptr, _stream
+from .op import _CALLS, _c, _device_of, _native, _ptr, _stream
 
 
 def angles_to_cos_sin(angles: torch.Tensor, dt: torch.Tensor,
@@ -375,6 +375,10 @@ def mamba3_scan(q, k, v, adt, dt, trap, q_bias, k_bias, angles=None,
     q_bias, k_bias : (h, dqk); D : (h,)
     returns : (b, l, h, dv) [, last_state (b, h, dv, dqk), last_bx (b, h, dqk)]
     """
+    r = _native("mamba3", q, k, v, adt, dt, trap, q_bias, k_bias, cos, sin, angles, D, z, None,
+                None, None, bool(reverse), bool(return_last_state), False)
+    if r is not None:
+        return r
     if q.dim() == 3:
         q = q.unsqueeze(2)
     if k.dim() == 3:
@@ -432,6 +436,10 @@ def mamba3_mimo_scan(q, k, v, adt, dt, trap, q_bias, k_bias, psi, zeta, phi,
     MIMO rotates split-halves pairs (i, i + dqk/2), SISO interleaved pairs
     (2i, 2i+1): a rank-1 MIMO call equals a SISO call only without rotation.
     """
+    r = _native("mamba3", q, k, v, adt, dt, trap, q_bias, k_bias, cos, sin, angles, D, z, psi,
+                zeta, phi, bool(reverse), bool(return_last_state), True)
+    if r is not None:
+        return r
     if q.dim() == 4:
         q = q.unsqueeze(3)
     if k.dim() == 4:

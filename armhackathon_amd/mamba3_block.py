@@ -32,7 +32,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ffi
-from .op import _CALLS, _device_of, _stream
+from .op import _CALLS, _device_of, _native, _stream
 
 
 def heavy_tail_activation(x: torch.Tensor) -> torch.Tensor:
@@ -186,12 +186,15 @@ class Mamba3Mixer(nn.Module):
         proj = F.linear(u, self.in_proj.weight)
         proj = proj.to(torch.float32).contiguous()
         mimo = self.is_mimo
-        y = _mixer_scan_op(
+        args = (
             proj, _f32(self.dt_bias), _f32(self.B_norm.weight), _f32(self.C_norm.weight),
             _f32(self.B_bias), _f32(self.C_bias), _f32(self.D),
             _f32(self.mimo_x) if mimo else None, _f32(self.mimo_z) if mimo else None,
             _f32(self.mimo_o) if mimo else None, self.nheads, self.headdim, self.d_state,
             self.mimo_rank, self.num_bc_heads, self.num_rope_angles, float(self.A_floor),
             float(self.B_norm.eps))
+        y = _native("mixer_scan", *args)
+        if y is None:
+            y = _mixer_scan_op(*args)
         y = y.reshape(b, seqlen, self.nheads * self.headdim)
         return self.out_proj(y.to(u.dtype))

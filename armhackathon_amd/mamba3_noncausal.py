@@ -27,7 +27,7 @@ import torch
 
 from . import _ffi
 from .mamba3 import _check_shapes, _cos_sin
-from .op import _CALLS, _c, _device_of, _ptr, _stream
+from .op import _CALLS, _c, _device_of, _native, _ptr, _stream
 from .ss2d import _MERGES, grid_to_views
 from .ss2d_mamba3 import _check_grid, grid_to_views_time_major, views_to_grid_time_major
 
@@ -81,6 +81,9 @@ def noncausal_scan(q, k, v, adt, dt, trap, q_bias, k_bias, angles=None,
     q, k (b, l, g, dqk) or (b, l, dqk); the other arguments as for `mamba3_scan`.
     The angle pre-pass runs once and serves both traversals.
     """
+    r = _native("noncausal", q, k, v, adt, dt, trap, q_bias, k_bias, cos, sin, angles, D, z)
+    if r is not None:
+        return r
     if q.dim() == 3:
         q = q.unsqueeze(2)
     if k.dim() == 3:

@@ -10,6 +10,11 @@ the tensors' device, and the call returns without synchronising. A host tensor
 is an error, not a cue to fall back: this package has no CPU implementation.
 
 Inference-only, like the reference: no autograd formula is registered.
+
+A plain eager call (float32 device tensors, no gradient to record, no transform or mode in
+between) goes through the native front-end (`_front.py`) instead of the custom op: the same
+checks and the same kernels, a third of the host time. Everything else, and every refusal,
+is the custom op's.
 """
 
 from typing import Optional, Tuple
@@ -17,6 +22,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _ffi
+from ._front import front
 
 _CALLS = {"n": 0}
 
@@ -47,6 +53,17 @@ def _device_of(*tensors):
 
 def _stream(dev):
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+def _native(name, *args):
+    """The native front-end's result, or None: the call is not the plain one it serves."""
+    f = front()
+    if f is None:
+        return None
+    r = getattr(f, name)(*args)
+    if r is not None:
+        _CALLS["n"] += 1
+    return r
 
 
 def _check_m1(u, delta, a, b, c, d_skip, z, delta_bias, h0):
@@ -127,6 +144,10 @@ def selective_scan(u, delta, A, B, C, D=None, z=None, delta_bias=None,
     unchanged (timestep t still lands at index t); under reverse, last_state
     is the state after consuming t = 0.
     """
+    r = _native("selective_scan", u, delta, A, B, C, D, z, delta_bias, initial_state,
+                bool(delta_softplus), bool(reverse))
+    if r is not None:
+        return r if return_last_state else r[0]
     batch, dim, length = u.shape
     state = A.shape[1]
     B = _bc4(B, batch, state, length)
@@ -223,6 +244,10 @@ def selective_scan_time_major(u, delta, A, B, C, D=None, z=None, delta_bias=None
     mixer's out_proj. Same arguments, values and final state as `selective_scan`.
     The reference copies z here (python/arm_scan/op.py:19-20); this has no
     counterpart there."""
+    r = _native("selective_scan_time_major", u, delta, A, B, C, D, z, delta_bias,
+                initial_state, bool(delta_softplus), bool(reverse))
+    if r is not None:
+        return r if return_last_state else r[0]
     batch, dim, length = u.shape
     state = A.shape[1]
     B = _bc4(B, batch, state, length)
@@ -288,6 +313,9 @@ def selective_state_update(state, x, dt, A, B, C, D=None, z=None, dt_bias=None,
     strided views (they are read in place); A (dim, N); D, dt_bias (dim,). The
     semantics of transformers' mamba_selective_state_update, in one kernel; the
     reference has no counterpart (it leaves decoding to upstream, README.md:320-322)."""
+    y = _native("state_update", state, x, dt, A, B, C, D, z, dt_bias, bool(dt_softplus))
+    if y is not None:
+        return y
     f = lambda t: None if t is None else (t if t.dtype == torch.float32 else t.float())
     return _state_update_op(state, f(x), f(dt), _c(A), f(B), f(C),
                             None if D is None else _c(D), f(z),
@@ -331,6 +359,9 @@ def selective_scan_bidirectional(u, delta, A, B, C, D=None, z=None,
     """Forward and reverse scans of the same inputs in one call
     (python/arm_scan/op.py:138-160) -> (out_fwd, out_bwd), through
     arm_scan_selective_scan_bidirectional_f32 (its routes: include/arm_scan_hip.h)."""
+    r = _native("bidirectional", u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus))
+    if r is not None:
+        return r
     batch, dim, length = u.shape
     state = A.shape[1]
     B = _bc4(B, batch, state, length)
@@ -405,6 +436,9 @@ def causal_conv1d(x, weight, bias=None, activation=None, time_major=False):
     transpose (and the scan reads in place)."""
     if activation not in (None, "silu", "swish"):
         raise ValueError(f"activation must be None or 'silu', got {activation!r}")
+    y = _native("causal_conv1d", x, weight, bias, activation is not None, bool(time_major))
+    if y is not None:
+        return y
     if x.dim() != 3 or weight.dim() != 2 or weight.shape[0] != x.shape[1]:
         raise ValueError(f"x (batch, dim, len) and weight (dim, width) expected, got "
                          f"{tuple(x.shape)} and {tuple(weight.shape)}")
@@ -442,6 +476,9 @@ def causal_conv1d_update(x, conv_state, weight, bias=None, activation=None):
     read in place); returns (batch, dim) = act(bias + weight . window)."""
     if activation not in (None, "silu", "swish"):
         raise ValueError(f"activation must be None or 'silu', got {activation!r}")
+    y = _native("causal_conv1d_update", x, conv_state, weight, bias, activation is not None)
+    if y is not None:
+        return y
     if x.dim() != 2 or weight.dim() != 2 or weight.shape[0] != x.shape[1]:
         raise ValueError(f"x (batch, dim) and weight (dim, width) expected, got "
                          f"{tuple(x.shape)} and {tuple(weight.shape)}")

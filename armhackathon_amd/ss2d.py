@@ -17,7 +17,7 @@ view-based composition over the bidirectional scan instead.
 import torch
 
 from . import _ffi
-from .op import _CALLS, _c, _device_of, _ptr, _stream
+from .op import _CALLS, _c, _device_of, _native, _ptr, _stream
 
 _MERGES = ("sum", "mean", "none")
 
@@ -122,6 +122,12 @@ def ss2d_scan(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=True,
                           ("z", z, (b, d, h, w))):
         if t is not None and tuple(t.shape) != want:
             raise ValueError(f"{name} must be {want}, got {tuple(t.shape)}")
+    r = _native("ss2d", u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus),
+                _ffi.SS2D_MERGES[merge], bool(return_last_state))
+    if r is not None:
+        out, last = r
+        res = tuple(out.unbind(0)) if merge == "none" else out
+        return (res, last) if return_last_state else res
     dev = _device_of(u, delta, A, B, C, D, z, delta_bias)
     u, delta, A, B, C = _c(u), _c(delta), _c(A), _c(B), _c(C)
     D = None if D is None else _c(D)

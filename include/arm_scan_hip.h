@@ -26,6 +26,7 @@
  *       arm_scan_mamba3_noncausal_f32, the non-causal Mamba-3 sum;
  *       arm_scan_mamba3_block_frontend_f32 and arm_scan_mamba3_scan_strided_f32, the
  *         Mamba-3 mixer's front-end and the scan reading its projection in place;
+ *       arm_scan_thread_scratch, a caller's allocator for the scratch of its calls;
  *   - code 6 reports a HIP launch / device error; arm_scan_last_error() explains
  *     the most recent nonzero code on the calling thread.
  *
@@ -309,6 +310,15 @@ int arm_scan_ss2d_f32(const ArmSS2DDims* dims, const float* u, const float* delt
                       const float* a, const float* b4, const float* c4, const float* d_skip,
                       const float* z, const float* delta_bias, int delta_softplus, int merge,
                       float* out, float* last_states, void* stream);
+
+/* No reference counterpart: where the calling thread's next calls take their scratch from.
+ * `alloc(ctx, bytes)` returns device memory of the current device, 16-byte aligned, which
+ * the caller keeps until the call has returned and after that gives back in the order of
+ * the call's stream (NULL: out of memory, the call fails with code 6). Null `alloc`: the
+ * library's stream-ordered pool, as for every thread that never set one; calls on a stream
+ * that is being captured take the pool in any case. A caller sets it around a call:
+ * the setting is this thread's alone. */
+void arm_scan_thread_scratch(void* (*alloc)(void* ctx, size_t bytes), void* ctx);
 
 /* Human-readable reason for the last nonzero code returned on this thread. */
 const char* arm_scan_last_error(void);

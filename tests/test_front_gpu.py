@@ -1,0 +1,226 @@
+"""The native eager front-end (csrc/torch_front.cpp): a plain call has the bits of the
+custom op's, and whatever is not plain is left to the custom op, which records, refuses or
+raises as it did."""
+
+import pytest
+
+from util import case
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(*shape, seed=0, scale=1.0):
+    import torch
+
+    g = torch.Generator(device="cuda").manual_seed(seed + sum(shape))
+    return torch.randn(*shape, device="cuda", generator=g) * scale
+
+
+def _calls():
+    import torch
+    import torch.nn.functional as F
+
+    import armhackathon_amd as arm
+    from armhackathon_amd.mamba3_block import Mamba3Mixer
+
+    b, d, n, L = 2, 32, 16, 260
+    u, dl = _rand(b, d, L), _rand(b, d, L, seed=1) - 3
+    A, D, bias = -torch.rand(d, n, device="cuda"), _rand(d, seed=2), _rand(d, seed=3)
+    B, C, z = _rand(b, n, L, seed=4), _rand(b, n, L, seed=5), _rand(b, d, L, seed=6)
+    Bs = _rand(b, L, 40, seed=7)[..., 8:8 + n].transpose(1, 2)  # a projection's columns
+    tm = _rand(b, L, 2 * d, seed=8).transpose(1, 2)
+    h0 = _rand(b, d, n, seed=9)
+    kw = dict(D=D, z=z, delta_bias=bias, delta_softplus=True)
+    w, wb = _rand(d, 4, seed=10), _rand(d, seed=11)
+    calls = {
+        "scan": lambda: arm.selective_scan(u, dl, A, B, C, return_last_state=True,
+                                           initial_state=h0, **kw),
+        "scan_reverse_groups": lambda: arm.selective_scan(
+            u, dl, A, B.view(b, 1, n, L).repeat(1, 2, 1, 1), C.view(b, 1, n, L).repeat(1, 2, 1, 1),
+            reverse=True, delta_softplus=True),
+        "scan_views": lambda: arm.selective_scan(tm[:, :d], dl, A, Bs, C, z=tm[:, d:],
+                                                 delta_softplus=True),
+        "time_major": lambda: arm.selective_scan_time_major(
+            tm[:, :d], dl, A, Bs, C, D=D, z=tm[:, d:], delta_softplus=True,
+            return_last_state=True),
+        "bidir": lambda: arm.bidirectional_scan(u, dl, A, B, C, merge="none", **kw),
+        "conv": lambda: arm.causal_conv1d(tm[:, :d], w, wb, activation="silu", time_major=True),
+        "conv_plain": lambda: arm.causal_conv1d(u, w),
+    }
+
+    def steps():
+        cs, hs = _rand(b, d, 4, seed=12), _rand(b, d, n, seed=13)
+        x = arm.causal_conv1d_update(tm[:, :d, 3], cs, w, wb, activation="silu")
+        y = arm.selective_state_update(hs, x, dl[..., 0], A, Bs[..., 0], C[..., 0], D=D,
+                                       z=z[..., 0], dt_bias=bias, dt_softplus=True)
+        return x, y, cs, hs
+
+    calls["steps"] = steps
+    H = 7
+    grid = [_rand(b, d, H, H, seed=s) for s in (20, 21, 22)]
+    B4, C4 = _rand(4, b, n, H, H, seed=23), _rand(4, b, n, H, H, seed=24)
+    calls["ss2d"] = lambda: arm.ss2d_scan(grid[0], grid[1] - 3, A, B4, C4, D=D, z=grid[2],
+                                          per_direction=True, return_last_state=True)
+    calls["ss2d_none"] = lambda: arm.ss2d_scan(grid[0], grid[1] - 3, A, B4[0], C4[0],
+                                               merge="none")
+    h, dv, dqk, Lm = 4, 32, 64, 75
+    dt = F.softplus(_rand(b, h, Lm, seed=30) - 3)
+    args = [_rand(b, Lm, dqk, seed=31, scale=0.1), _rand(b, Lm, 1, dqk, seed=32, scale=0.1),
+            _rand(b, Lm, h, dv, seed=33), -0.5 * dt, dt, _rand(b, h, Lm, seed=34),
+            _rand(h, dqk, seed=35, scale=0.1), _rand(h, dqk, seed=36, scale=0.1)]
+    ang, zz, Dh = _rand(b, Lm, h, 16, seed=37), _rand(b, Lm, h, dv, seed=38), _rand(h, seed=39)
+    cos, sin = arm.angles_to_cos_sin(ang, dt, dqk // 2)
+    shared = _rand(b, Lm, 1, 16, seed=40).expand(b, Lm, h, 16)
+    odd = _rand(b * Lm * h * 16 + 1, seed=41)[1:].view(b, Lm, h, 16)  # off a 16-byte base
+    for name, kw3 in dict(cos=dict(cos=cos, sin=sin), cos_reverse=dict(cos=cos, sin=sin,
+                                                                       reverse=True),
+                          angles=dict(angles=ang), angles_reverse=dict(angles=ang, reverse=True),
+                          angles_shared=dict(angles=shared), angles_odd=dict(angles=odd),
+                          carry=dict(angles=ang, return_last_state=True)).items():
+        calls["m3_" + name] = lambda kw3=kw3: arm.mamba3_scan(*args, D=Dh, z=zz, **kw3)
+    m = list(args)
+    m[0], m[1] = _rand(b, Lm, 4, dqk, seed=42), _rand(b, Lm, 4, 2, dqk, seed=43)
+    m[0] = m[0].unsqueeze(3).repeat(1, 1, 1, 2, 1)
+    m[6], m[7] = _rand(h, 4, dqk, seed=44), _rand(h, 4, dqk, seed=45)
+    ranks = [_rand(h, 4, dv, seed=s) for s in (46, 47, 48)]
+    for name, kw3 in dict(cos=dict(cos=cos, sin=sin, return_last_state=True),
+                          angles=dict(angles=ang), shared=dict(angles=shared),
+                          reverse=dict(angles=ang, reverse=True)).items():
+        calls["mimo_" + name] = lambda kw3=kw3: arm.mamba3_mimo_scan(*m, *ranks, D=Dh, z=zz,
+                                                                     **kw3)
+    calls["noncausal"] = lambda: arm.noncausal_scan(*args, angles=ang, D=Dh, z=zz)
+    mixer = Mamba3Mixer(d_model=64, d_state=32, headdim=32).to("cuda").requires_grad_(False)
+    x = _rand(b, Lm, 64, seed=50)
+    calls["mixer"] = lambda: mixer(x)
+    return calls
+
+
+def test_same_bits_as_the_custom_op(monkeypatch):
+    import torch
+
+    from armhackathon_amd import op
+
+    flat = lambda r: list(r) if isinstance(r, tuple) else [r]  # noqa: E731
+    leaves = lambda r: [t for x in flat(r) for t in flat(x)]  # noqa: E731
+    served, calls = [], _calls()
+    real = op.front()  # the GPU is in use from here on
+    for name, call in calls.items():
+        case(f"front-end {name}")
+
+        class Spy:
+            def __getattr__(self, fn):
+                def run(*a):
+                    r = getattr(real, fn)(*a)
+                    served.append((name, fn, r is not None))
+                    return r
+                return run
+
+        monkeypatch.setattr(op, "front", lambda: Spy())
+        got = leaves(call())
+        monkeypatch.setattr(op, "front", lambda: None)
+        want = leaves(call())
+        assert len(got) == len(want)
+        for g, w in zip(got, want):
+            assert g.shape == w.shape and g.stride() == w.stride() and torch.equal(g, w), name
+    assert served and all(ok for _, _, ok in served), [s for s in served if not s[2]]
+
+
+def test_not_plain_is_left_alone():
+    import torch
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    import armhackathon_amd as arm
+    from armhackathon_amd import op
+
+    b, d, n, L = 1, 16, 8, 40
+    u, dl = _rand(b, d, L), _rand(b, d, L, seed=1)
+    A, B = -torch.rand(d, n, device="cuda"), _rand(b, n, L, seed=2)
+    f = op.front()
+
+    def native(u=u, dl=dl):
+        return f.selective_scan(u, dl, A, B, B, None, None, None, None, True, False)
+
+    assert native() is not None
+    for bad in (u.double(), u.cpu(), u[0], u[:, :, :0], u.clone().requires_grad_(), None, 3,
+                torch.nn.Parameter(u.clone())):
+        case(f"not plain: {type(bad).__name__}")
+        assert native(u=bad) is None
+    assert native(dl=dl[..., :-1]) is None
+    with torch.no_grad():
+        assert native(u=u.clone().requires_grad_()) is not None
+    with torch.inference_mode():
+        assert native() is not None
+
+    class Fn(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Disp(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Fn(), Disp()):
+        with mode:
+            assert native() is None
+    seen = []
+
+    def inner(x):
+        seen.append(native(u=x) is None)
+        return x
+
+    torch.vmap(inner)(u.unsqueeze(0))
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(native(u=torch.autograd.forward_ad.make_dual(u, u)) is None)
+    assert seen == [True, True]
+    with pytest.raises(ValueError):
+        arm.selective_scan(u, dl[..., :-1], A, B, B)
+    y = arm.selective_scan(u.clone().requires_grad_(), dl, A, B, B, delta_softplus=True)
+    with pytest.raises(RuntimeError):
+        y.sum().backward()
+
+
+def test_state_version_counts():
+    """The states written in place count as written, as an op that mutates them does."""
+    import torch
+
+    import armhackathon_amd as arm
+
+    s, x = torch.zeros(1, 16, 4, device="cuda"), _rand(1, 16)
+    before = s._version
+    arm.causal_conv1d_update(x, s, _rand(16, 4, seed=1))
+    assert s._version > before
+    h = torch.zeros(1, 16, 8, device="cuda")
+    before = h._version
+    arm.selective_state_update(h, x, x, -torch.rand(16, 8, device="cuda"), _rand(1, 8), _rand(1, 8))
+    assert h._version > before
+
+
+def test_scratch_during_capture():
+    """Captured with torch's graphs, a call takes its scratch from the library's pool; each
+    replay equals the eager result, with eager calls between that reuse torch's blocks."""
+    import torch
+
+    import armhackathon_amd as arm
+
+    b, d, n, L = 1, 32, 16, 1024  # few rows: the segment maps are scratch
+    u, dl = _rand(b, d, L), _rand(b, d, L, seed=1)
+    A, B = -torch.rand(d, n, device="cuda"), _rand(b, n, L, seed=2)
+    run = lambda: arm.selective_scan(u, dl, A, B, B, delta_softplus=True)  # noqa: E731
+    want = run().clone()
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        run()
+    torch.cuda.current_stream().wait_stream(st)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = run()
+    for i in range(4):
+        case(f"replay {i}")
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        torch.full((4096, 256), float(i), device="cuda")
+        assert torch.equal(run(), want)
