@@ -85,6 +85,13 @@ constexpr size_t kLdsBudget = 160 * 1024;
 constexpr int kMinSplitChunks = 64;
 constexpr int kMinSplitChunksRank1 = 256;
 constexpr int kFoldStages = 8;       // deepest DMA ring of the fold pass
+// Equal segments (at most half as many blocks as CUs): from this many chunks, of at least
+// this many each, folded in pieces of at least this many, and at most this many pieces in
+// all for the last segment's blocks to combine
+constexpr int kMinEqualChunks = 24;
+constexpr int kMinSegChunks = 4;
+constexpr int kMinPieceChunks = 4;
+constexpr int kMaxPieces = 24;
 
 // CUs of the current device (0 if unknown), looked up once per device.
 int device_cus() {
@@ -121,17 +128,20 @@ struct M3K {
   int vt, zt, at;            // and per step
   // SISO: no same-step term (gamma on M's diagonal, D x) and out += the result
   int accum;
-  // Sequences cut at chunk `split` (0: whole sequences): blocks [0, seg_blocks) run
-  // chunks [split, nchunks) from the state m3_fold_kernel left in `fold`,
-  // blocks [seg_blocks, 2 seg_blocks) run chunks [0, split) from zero.
-  int split, seg_blocks;
+  // Sequences cut into nseg segments (split 0, nseg 1: whole sequences): segment 0 is
+  // chunks [0, split), segment s >= 1 the seg_len chunks from split + (s - 1) seg_len, the
+  // last one to nchunks. Blocks [0, seg_blocks) run the last segment, the next seg_blocks
+  // the one before it, and so on; segment s >= 1 starts from the state that
+  // m3_fold_kernel left in `fold`, segment 0 from zero.
+  int split, seg_blocks, nseg, seg_len;
   float* fold;
   int skip_q;  // the stage holds no q section (m3_fold_kernel's): k's comes first
-  // The fold runs in nsub pieces of sub_len chunks, one block each (per sequence and dv
-  // slices): piece s leaves its state from zero in fold + s * nseq * dv * dqk (in the
+  // The fold covers the segments but the last, chunks [0, fold_end), in nsub pieces of
+  // sub_len chunks that do not straddle segments, one block each (per sequence and dv
+  // slices); segment s starts from the first s * seg_pieces of them. Piece s leaves its state from zero in fold + s * nseq * dv * dqk (in the
   // order the waves hold it, fold_off) and its decay (the product of its chunks'
   // e^{c_last}) in fold_decay[s * nseq + seq]; the resuming blocks combine them in order.
-  int nsub, sub_len;
+  int nsub, sub_len, fold_end, seg_pieces;
   float* fold_decay;
   // With the fused angle pre-pass (SISO): fold piece s rotates its keys by theta
   // relative to its first step and leaves theta's increment over its steps (turns,
@@ -570,17 +580,17 @@ __global__ void __launch_bounds__(64 * (kMaxWaves + 4)) m3_chunk_kernel(M3K p) {
   const int ej = ewave ? (wave - WN) % PT : 0;      // slice of an epilogue wave
   const int epar = ewave ? (wave - WN) / PT : 0;    // chunk parity of an epilogue wave
   const int li = lane & 15, lj = lane >> 4;
-  // this block's chunks [cb, ce): the tail segment (from the folded state) comes first
-  // in block order, so that its longer blocks start first; the head segment's blocks
-  // fill the CUs left over, several in turn
-  int bid = blockIdx.x, cb = 0, ce = p.nchunks;
+  // this block's chunks [cb, ce): the last segment comes first in block order, so that
+  // where the first segment is the shorter one (two segments) the longer blocks start
+  // first and the others fill the CUs left over, several in turn
+  int bid = blockIdx.x, cb = 0, ce = p.nchunks, pieces = 0;
   if (p.split) {
-    if (bid >= p.seg_blocks) {
-      bid -= p.seg_blocks;
-      ce = p.split;
-    } else {
-      cb = p.split;
-    }
+    const int g = bid / p.seg_blocks;
+    const int seg = p.nseg - 1 - g;
+    bid -= g * p.seg_blocks;
+    if (seg > 0) cb = p.split + (seg - 1) * p.seg_len;
+    if (g > 0) ce = seg > 0 ? cb + p.seg_len : p.split;
+    pieces = seg * p.seg_pieces;
   }
   // blocks of one sequence share an XCD (block id mod 8), and so its L2
   const int bx = bid & 7, by = bid >> 3;
@@ -805,9 +815,9 @@ __global__ void __launch_bounds__(64 * (kMaxWaves + 4)) m3_chunk_kernel(M3K p) {
   // fused angles: theta before the chunk of the pairs the lane computes (SISO: pairs
   // 8nt + 2lj + e)
   float carry[2] = {0.0f, 0.0f};       // SISO: 2 per lane
-  // resuming at chunk cb = split: the head segment's state, its pieces in order, and
+  // resuming at chunk cb > 0: the state there, from the pieces before it in order, and
   // with fused angles theta there, the pieces' increments summed
-  for (int sb = 0; cb > 0 && sb < p.nsub; ++sb) {
+  for (int sb = 0; sb < pieces; ++sb) {
     const float dcy = p.fold_decay[sb * p.nseq + seq];
     const float* fold = p.fold + (long long)sb * p.nseq * dv * dqk;
     float c0 = 1.0f, s0 = 0.0f, c1 = 1.0f, s1 = 0.0f;
@@ -1057,10 +1067,10 @@ __global__ void __launch_bounds__(64 * (kMaxWaves + 4)) m3_chunk_kernel(M3K p) {
   }
 }
 
-// The state a sequence reaches after its chunks [0, p.split), from zero, written to
-// p.fold (in fold_off's order): the partial waves' state update alone (no q, no outputs, no
-// epilogue waves), S = e^{c_last} S + K^T diag(w) X per chunk, for the blocks of
-// m3_chunk_kernel that resume at chunk p.split. Its stage is the scan's without q and z
+// What each piece of a sequence's chunks [0, p.fold_end) does to the state, from zero,
+// written to p.fold (in fold_off's order): the partial waves' state update alone (no q, no
+// outputs, no epilogue waves), S = e^{c_last} S + K^T diag(w) X per chunk, for the blocks
+// of m3_chunk_kernel that resume at a later segment. Its stage is the scan's without q and z
 // (the host builds this kernel's M3K so: skip_q), about 20 KB at config 3, so that a
 // ring of up to kFoldStages stages keeps 7 chunks of DMA in flight: the pass does little
 // work per chunk, and with the scan's 3 chunks ahead it waited on memory. K is
@@ -1072,7 +1082,7 @@ __global__ void __launch_bounds__(64 * kMaxWaves) m3_fold_kernel(M3K p) {
   const int lane = threadIdx.x & 63;
   const int nt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int li = lane & 15, lj = lane >> 4;
-  const int sub = blockIdx.x / p.seg_blocks;  // this block's piece of the head segment
+  const int sub = blockIdx.x / p.seg_blocks;  // this block's piece
   const int bid = blockIdx.x - sub * p.seg_blocks;
   const int bx = bid & 7, by = bid >> 3;
   const int nb = p.nparts / PT;
@@ -1087,9 +1097,9 @@ __global__ void __launch_bounds__(64 * kMaxWaves) m3_fold_kernel(M3K p) {
   const int n0 = nt * 16 + 4 * lj;
   const bool lo = !MIMO || n0 < half;
   const int step_i = li / R;
-  // chunks [cb, ce) of the head segment [0, split), all whole (split < L / T)
+  // chunks [cb, ce) of [0, fold_end), all whole (fold_end < nchunks)
   const int cb = sub * p.sub_len;
-  const int ce = cb + p.sub_len < p.split ? cb + p.sub_len : p.split;
+  const int ce = cb + p.sub_len < p.fold_end ? cb + p.sub_len : p.fold_end;
   float* stages = sm;
   float* kt = stages + NS * p.stage_floats + nt * 16 * kKtStride;
   const int off_k = 0, off_cs = WN * 256;
@@ -1283,35 +1293,44 @@ size_t fold_lds_bytes(const M3K& k, int ns) {
 // Blocks of the fold kernel kf launches that one CU holds at once with `lds` bytes of LDS
 // each: its registers limit them as well as its LDS (the rank-4 MIMO fold's 88 VGPRs
 // allow five waves a SIMD, so two blocks of eight waves a CU where LDS would allow three).
-template <int R, bool MIMO>
-int fold_resident(const M3K& kf, size_t lds, bool narrow) {
-  int n = 0;
-  auto occ = [&](const void* kernel) {
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 64 * (kf.dqk / 16), lds) !=
-        hipSuccess) {
-      (void)hipGetLastError();
-      n = 1;
-    }
-  };
-  const int pt = kf.ptiles;
-  if (narrow) {
-    if (pt == 4) occ(reinterpret_cast<const void*>(&m3_fold_kernel<R, MIMO, false, 4, kNarrowDma>));
-    else if (pt == 2) occ(reinterpret_cast<const void*>(&m3_fold_kernel<R, MIMO, false, 2, kNarrowDma>));
-    else occ(reinterpret_cast<const void*>(&m3_fold_kernel<R, MIMO, false, 1, kNarrowDma>));
-  } else {
-    if (pt == 4) occ(reinterpret_cast<const void*>(&m3_fold_kernel<R, MIMO, false, 4, kMaxDma>));
-    else if (pt == 2) occ(reinterpret_cast<const void*>(&m3_fold_kernel<R, MIMO, false, 2, kMaxDma>));
-    else occ(reinterpret_cast<const void*>(&m3_fold_kernel<R, MIMO, false, 1, kMaxDma>));
+// The registers' share is asked of the runtime once per kernel and block size (the query
+// took 8 us of a call) and kept: it is a property of the compiled kernel.
+template <int R, bool MIMO, int PT, int MD>
+int fold_resident_regs(const M3K& kf) {
+  static std::atomic<int> cache[kMaxWaves + 1];  // by waves a block
+  const int wn = kf.dqk / 16;
+  int n = cache[wn].load(std::memory_order_relaxed);
+  if (n > 0) return n;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+          &n, reinterpret_cast<const void*>(&m3_fold_kernel<R, MIMO, false, PT, MD>), 64 * wn,
+          0) != hipSuccess) {
+    (void)hipGetLastError();
+    return 1;  // asked again by the next call
   }
+  cache[wn].store(n < 1 ? 1 : n, std::memory_order_relaxed);
   return n;
 }
 
+template <int R, bool MIMO>
+int fold_resident(const M3K& kf, bool narrow) {
+  const int pt = kf.ptiles;
+  if (narrow)
+    return pt == 4   ? fold_resident_regs<R, MIMO, 4, kNarrowDma>(kf)
+           : pt == 2 ? fold_resident_regs<R, MIMO, 2, kNarrowDma>(kf)
+                     : fold_resident_regs<R, MIMO, 1, kNarrowDma>(kf);
+  return pt == 4   ? fold_resident_regs<R, MIMO, 4, kMaxDma>(kf)
+         : pt == 2 ? fold_resident_regs<R, MIMO, 2, kMaxDma>(kf)
+                   : fold_resident_regs<R, MIMO, 1, kMaxDma>(kf);
+}
+
 int fold_resident_any(const M3K& kf, size_t lds, bool narrow) {
-  if (kf.psi == nullptr) return fold_resident<1, false>(kf, lds, narrow);
+  const int by_lds = (int)(kLdsBudget / lds);
   const int R = 16 / kf.steps_per_chunk;
-  if (R == 1) return fold_resident<1, true>(kf, lds, narrow);
-  if (R == 2) return fold_resident<2, true>(kf, lds, narrow);
-  return fold_resident<4, true>(kf, lds, narrow);
+  const int by_regs = kf.psi == nullptr ? fold_resident<1, false>(kf, narrow)
+                      : R == 1          ? fold_resident<1, true>(kf, narrow)
+                      : R == 2          ? fold_resident<2, true>(kf, narrow)
+                                        : fold_resident<4, true>(kf, narrow);
+  return by_lds < by_regs ? by_lds : by_regs;
 }
 
 template <int R, bool MIMO, int PT, int MD>
@@ -1327,7 +1346,7 @@ hipError_t launch_fold(const M3K& kf, bool rev, hipStream_t st) {
 template <int R, bool MIMO, int PT, bool ZOWN, int MD>
 hipError_t launch_chunk(const M3K& k, bool rev, hipStream_t st) {
   const int WN = k.dqk / 16;
-  const long long blocks = 8LL * (k.nparts / PT) * ((k.nseq + 7) / 8) * (k.split ? 2 : 1);
+  const long long blocks = 8LL * (k.nparts / PT) * ((k.nseq + 7) / 8) * k.nseg;
   const size_t lds = chunk_lds_bytes(k, PT, k.nstages);
   if (k.ang) {  // forward only: theta is a forward cumsum
     if (rev) return hipErrorInvalidValue;
@@ -1362,7 +1381,7 @@ hipError_t launch_chunk_pt(const M3K& k, const M3K& kf, bool rev, hipStream_t st
   auto go = [&](auto zown, auto md) {
     constexpr bool Z = decltype(zown)::value;
     constexpr int M = decltype(md)::value;
-    if (k.split) {
+    if (k.nseg > 1) {
       const hipError_t e = kf.ptiles == 4   ? launch_fold<R, MIMO, 4, M>(kf, rev, st)
                            : kf.ptiles == 2 ? launch_fold<R, MIMO, 2, M>(kf, rev, st)
                                             : launch_fold<R, MIMO, 1, M>(kf, rev, st);
@@ -1441,34 +1460,57 @@ hipError_t m3_scan_chunked(const M3Problem& pr, hipStream_t st) {
   if (k.n_ins > kMaxDma * WN) return hipErrorInvalidValue;  // DMA by the WN partial waves
 
   // Too few sequences for the chip. A block takes a whole CU (its LDS), so with P
-  // blocks on C > P CUs, C - P CUs idle through the scan. Each sequence is then cut at
-  // chunk `split`: a fold pass first computes the state every sequence reaches there
-  // (the state update alone), then the scan runs 2P blocks, the P that resume at
-  // `split` first and the P head segments [0, split) after them, several in turn on
-  // the CUs the first P leave free. With deep = ceil(P / (C - P)) head segments per
-  // free CU, each paying its ring's fill and drain (about 2 NS chunks), split =
-  // (nchunks - 2 NS (deep - 1)) / (deep + 1) ends both groups together (configs 3 and
-  // 4: 192 blocks on 256 CUs, deep 3, split near a quarter). The fold costs about 0.7
-  // of a scan chunk per chunk at rank 1 and 0.4 at rank 4 (rank-4 chunks hold 4 steps
-  // whose state update is a quarter of their work), so rank 1 splits from 256 chunks
-  // (measured at B4 H24 against whole sequences: L 2048 +5%, 4096 -2%, 8192 -7%) and
-  // other ranks from 64 (rank 4: L 1024 -5%, 2048 -11%, 4096 -14%, 8192 -16%). With the
-  // fused angle pre-pass (SISO) the fold pieces rotate by theta from their own start and
-  // the resuming blocks rotate each piece's state by theta at the piece's start (the
-  // pieces' increments summed); MIMO keeps whole sequences.
+  // blocks on C > P CUs, C - P CUs idle through the scan. Each sequence is then cut into
+  // segments: a fold pass first computes what the chunks before each cut do to the state
+  // (the state update alone, in pieces, many at once), then the scan runs every segment's
+  // blocks, each starting from the pieces before it.
+  //
+  // Up to C / 2 blocks: floor(C / P) equal segments, so that all blocks run at once. Rank
+  // 1, H24 dv64 dqk128, one sequence of L (time of a call): L 512 50 -> 37 us, 1024 86 -> 54,
+  // 2048 158 -> 78, 4096 187 -> 120; rank 4: L 128 47 -> 34, 512 100 -> 72; rank 4 and 8
+  // heads of L 512 112 -> 41. The fold pass and a second start of the ring cost about 12
+  // us, so the cuts start at 24 chunks (16: 33 against 31 us of kernels, less than the
+  // extra launch costs a caller who is behind the GPU).
+  //
+  // More than C / 2: one cut at chunk `split`. The P blocks that resume there come first
+  // and the P head segments [0, split) after them, several in turn on the CUs the first P
+  // leave free. With deep = ceil(P / (C - P)) head segments per free CU, each paying its
+  // ring's fill and drain (about 2 NS chunks), split = (nchunks - 2 NS (deep - 1)) /
+  // (deep + 1) ends both groups together (configs 3 and 4: 192 blocks on 256 CUs, deep 3,
+  // split near a quarter). The fold costs about 0.7 of a scan chunk per chunk at rank 1 and
+  // 0.4 at rank 4 (rank-4 chunks hold 4 steps whose state update is a quarter of their
+  // work), so rank 1 splits from 256 chunks (measured at B4 H24 against whole sequences: L
+  // 2048 +5%, 4096 -2%, 8192 -7%) and other ranks from 64 (rank 4: L 1024 -5%, 2048 -11%,
+  // 4096 -14%, 8192 -16%).
+  //
+  // With the fused angle pre-pass (SISO) the fold pieces rotate by theta from their own
+  // start and the resuming blocks rotate each piece's state by theta at the piece's start
+  // (the pieces' increments summed); MIMO keeps whole sequences.
   M3K kf = k;
   const long long blocks = (long long)k.nseq * (k.nparts / k.ptiles);
   const int cus = device_cus();
   const int min_chunks = R == 1 ? kMinSplitChunksRank1 : kMinSplitChunks;
-  if ((!pr.angles || !k.psi) && cus > 0 && blocks < cus && k.nchunks >= min_chunks &&
+  k.nseg = 1;
+  if ((!pr.angles || !k.psi) && cus > 0 && blocks < cus &&
       2 * chunk_lds_bytes(k, k.ptiles, k.nstages) > kLdsBudget) {
-    const long long deep = (blocks + (cus - blocks) - 1) / (cus - blocks);
-    const int split =
-        (int)((k.nchunks - 2LL * k.nstages * (deep - 1)) / (deep + 1));
-    if (split >= kMinSplitChunks / 4 && split < k.len / k.steps_per_chunk) {
-      k.split = split;
+    if (2 * blocks <= cus) {
+      long long nseg = cus / blocks;
+      if (nseg > k.nchunks / kMinSegChunks) nseg = k.nchunks / kMinSegChunks;
+      if (k.nchunks >= kMinEqualChunks && nseg >= 2) {
+        k.seg_len = k.split = (int)((k.nchunks + nseg - 1) / nseg);
+        k.nseg = (k.nchunks + k.seg_len - 1) / k.seg_len;
+      }
+    } else if (k.nchunks >= min_chunks) {
+      const long long deep = (blocks + (cus - blocks) - 1) / (cus - blocks);
+      const int split =
+          (int)((k.nchunks - 2LL * k.nstages * (deep - 1)) / (deep + 1));
+      if (split >= kMinSplitChunks / 4 && split < k.len / k.steps_per_chunk) {
+        k.split = split;
+        k.nseg = 2;
+      }
+    }
+    if (k.nseg > 1) {
       k.seg_blocks = 8 * (k.nparts / k.ptiles) * ((k.nseq + 7) / 8);
-      kf.split = split;
       kf.z = nullptr;  // the fold's stage: the scan's without q and z
       kf.zown = 0;
       kf.n_z = 0;
@@ -1488,42 +1530,51 @@ hipError_t m3_scan_chunked(const M3Problem& pr, hipStream_t st) {
       const long long fblocks = (long long)k.nseq * (k.nparts / kf.ptiles);
       // up to three fold blocks per CU, as many as the CU holds with a ring of two stages
       // (a shallow ring each: latency is covered by the other blocks' waves; LDS and
-      // registers both limit them), and the head segment in as many pieces as keep every
-      // fold block resident at once: a second round of blocks would double the pass
+      // registers both limit them), and the folded segments in as many pieces as keep
+      // every fold block resident at once: a second round of blocks would double the pass
       // (config 3: two blocks per CU, five pieces of 12 chunks, 480 blocks; eight pieces,
       // 768 blocks, ran in two rounds)
       const bool narrow = k.n_ins <= kNarrowDma * WN;  // the DMA plan launch_chunk_pt takes
-      int bpc = 3;
-      while (bpc > 1 && (bpc * fold_lds_bytes(kf, 2) > kLdsBudget ||
-                         fold_resident_any(kf, fold_lds_bytes(kf, 2), narrow) < bpc))
-        --bpc;
+      int bpc = fold_resident_any(kf, fold_lds_bytes(kf, 2), narrow);
+      bpc = bpc > 3 ? 3 : bpc < 1 ? 1 : bpc;
       kf.nstages = kFoldStages;
       while (kf.nstages > 2 && bpc * fold_lds_bytes(kf, kf.nstages) > kLdsBudget) --kf.nstages;
-      int nsub = (int)(bpc * (long long)cus / fblocks);
-      nsub = nsub < 1 ? 1 : nsub > split ? split : nsub;
-      k.sub_len = kf.sub_len = (split + nsub - 1) / nsub;
-      k.nsub = kf.nsub = (split + k.sub_len - 1) / k.sub_len;
+      const int folded = k.nseg - 1;  // segments the fold covers
+      int per_seg = (int)(bpc * (long long)cus / (fblocks * folded));
+      if (k.nseg > 2) {
+        if (per_seg > kMaxPieces / folded) per_seg = kMaxPieces / folded;
+        if (per_seg > k.split / kMinPieceChunks) per_seg = k.split / kMinPieceChunks;
+      }
+      per_seg = per_seg < 1 ? 1 : per_seg > k.split ? k.split : per_seg;
+      k.sub_len = (k.split + per_seg - 1) / per_seg;
+      k.seg_pieces = (k.split + k.sub_len - 1) / k.sub_len;
+      if (k.nseg > 2) {  // every segment whole pieces
+        k.seg_len = k.split = k.seg_pieces * k.sub_len;
+        k.nseg = (k.nchunks + k.seg_len - 1) / k.seg_len;
+      }
+      k.nsub = (k.nseg - 1) * k.seg_pieces;
+      k.fold_end = k.split + (k.nseg - 2) * k.seg_len;
+      kf.split = k.split;
+      kf.nsub = k.nsub;
+      kf.sub_len = k.sub_len;
+      kf.fold_end = k.fold_end;
       kf.seg_blocks = 8 * (k.nparts / kf.ptiles) * ((k.nseq + 7) / 8);
     }
   }
 
+  // One scratch block: the gate records, then the fold's states, decays and angles.
   const size_t nrec = (size_t)k.nseq * k.nchunks;
-  hipError_t e = stream_alloc((void**)&k.rec, nrec * k.rec_floats * sizeof(float), st);
+  const size_t rs = nrec * k.rec_floats;  // whole 16-byte pieces
+  const size_t fs = k.nseg > 1 ? (size_t)k.nsub * k.nseq * k.dv * k.dqk : 0;
+  const size_t ds = k.nseg > 1 ? (size_t)k.nsub * k.nseq : 0;
+  const size_t ts = k.ang ? ds * 64 : 0;
+  hipError_t e = stream_alloc((void**)&k.rec, (rs + fs + ds + ts) * sizeof(float), st);
   if (e != hipSuccess) return e;
   kf.rec = k.rec;
-  if (k.split) {
-    const size_t fs = (size_t)k.nsub * k.nseq * k.dv * k.dqk;
-    const size_t ds = (size_t)k.nsub * k.nseq, ts = k.ang ? ds * 64 : 0;
-    e = stream_alloc((void**)&k.fold, (fs + ds + ts) * sizeof(float), st);
-    if (e != hipSuccess) {
-      (void)stream_free(k.rec, st);
-      return e;
-    }
-    k.fold_decay = k.fold + fs;
-    k.theta = k.ang ? k.fold_decay + ds : nullptr;
-    kf.fold = k.fold;
-    kf.fold_decay = k.fold_decay;
-    kf.theta = k.theta;
+  if (k.nseg > 1) {
+    kf.fold = k.fold = k.rec + rs;
+    kf.fold_decay = k.fold_decay = k.fold + fs;
+    kf.theta = k.theta = k.ang ? k.fold_decay + ds : nullptr;
   }
   const unsigned gblocks = (unsigned)((nrec + 16 * R - 1) / (16 * R));  // 16R records a block
   const int rev = pr.reverse ? 1 : 0;
@@ -1538,11 +1589,7 @@ hipError_t m3_scan_chunked(const M3Problem& pr, hipStream_t st) {
     else if (R == 2) e = launch_chunk_pt<2, true>(k, kf, rev, st);
     else e = launch_chunk_pt<4, true>(k, kf, rev, st);
   }
-  hipError_t fe = stream_free(k.rec, st);
-  if (k.fold) {
-    const hipError_t fe2 = stream_free(k.fold, st);
-    if (fe == hipSuccess) fe = fe2;
-  }
+  const hipError_t fe = stream_free(k.rec, st);
   return e != hipSuccess ? e : fe;
 }
 
