@@ -103,6 +103,19 @@ def _declare(lib):
                   _vp, _vp,              # out out_strides
                   _vp, _vp,              # last_state h0
                   _vp]                   # stream
+    f = lib.arm_scan_selective_scan_views_f32
+    f.restype = _ci
+    f.argtypes = [ctypes.POINTER(ArmScanDims),
+                  _vp, _vp, _vp, _vp,    # u u_strides delta a
+                  _vp, _vp, _vp, _vp,    # b b_strides c c_strides
+                  _vp, _vp, _vp, _vp,    # d_skip z z_strides delta_bias
+                  _ci, _ci,              # delta_softplus reverse
+                  _vp, _vp,              # out out_strides
+                  _vp, _vp,              # last_state h0
+                  _vp]                   # stream
+    f = lib.arm_scan_thread_scratch
+    f.restype = None
+    f.argtypes = [_vp, _vp]              # alloc ctx
     f = lib.arm_scan_selective_state_update_f32
     f.restype = _ci
     f.argtypes = [*([ctypes.c_size_t] * 3),      # batch dim state_dim

@@ -15,7 +15,7 @@ import torch
 
 from . import _ffi
 
-_FUNCTIONS = ("arm_scan_selective_scan_f32", "arm_scan_selective_scan_strided_f32",
+_FUNCTIONS = ("arm_scan_selective_scan_f32", "arm_scan_selective_scan_views_f32",
               "arm_scan_selective_state_update_f32",
               "arm_scan_selective_scan_bidirectional_f32",
               "arm_scan_mamba3_scan_time_major_f32", "arm_scan_mamba3_scan_angles_f32",

@@ -309,6 +309,40 @@ int arm_scan_selective_scan_strided_f32(const ArmScanDims* dims, const float* u,
   return run(armscan::m1_scan(p, (hipStream_t)stream), "selective_scan (strided) launch");
 }
 
+int arm_scan_selective_scan_views_f32(
+    const ArmScanDims* dims, const float* u, const long long* u_strides, const float* delta,
+    const float* a, const float* b, const long long* b_strides, const float* c,
+    const long long* c_strides, const float* d_skip, const float* z, const long long* z_strides,
+    const float* delta_bias, int delta_softplus, int reverse, float* out,
+    const long long* out_strides, float* last_state, const float* h0, void* stream) {
+  if (!dims || !u || !delta || !a || !b || !c || !out)
+    return fail(ARM_SCAN_ERR_NULL_POINTER, "a required pointer is null");
+  if (int rc = check_m1_dims(*dims)) return rc;
+  armscan::M1Problem p{};
+  p.batch = dims->batch; p.dim = dims->dim; p.len = dims->len; p.state = dims->state;
+  p.groups = dims->groups;
+  p.u = u; p.delta = delta; p.A = a; p.B = b; p.C = c; p.D = d_skip; p.z = z;
+  p.bias = delta_bias; p.h0 = h0; p.out = out; p.last = last_state;
+  p.softplus = delta_softplus != 0; p.reverse = reverse != 0;
+  const long long L = (long long)dims->len, N = (long long)dims->state;
+  const long long cont[3] = {(long long)dims->dim * L, L, 1};
+  const long long bc[4] = {(long long)dims->groups * N * L, N * L, L, 1};
+  p.has_strides = 1;
+  p.views = 1;
+  for (int i = 0; i < 4; ++i) {
+    if (i < 3) {
+      p.z_stride[i] = z_strides ? z_strides[i] : cont[i];
+      p.out_stride[i] = out_strides ? out_strides[i] : cont[i];
+      p.u_stride[i] = u_strides ? u_strides[i] : cont[i];
+    }
+    p.b_stride[i] = b_strides ? b_strides[i] : bc[i];
+    p.c_stride[i] = c_strides ? c_strides[i] : bc[i];
+  }
+  const char* why = nullptr;
+  if (!armscan::m1_strided_supported(p, &why)) return fail(ARM_SCAN_ERR_INVALID_DIMS, "%s", why);
+  return run(armscan::m1_scan(p, (hipStream_t)stream), "selective_scan (views) launch");
+}
+
 int arm_scan_selective_state_update_f32(
     size_t batch, size_t dim, size_t state_dim, float* state, const float* x,
     const long long* x_strides, const float* dt, const long long* dt_strides, const float* a,

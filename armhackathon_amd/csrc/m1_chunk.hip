@@ -704,8 +704,10 @@ __device__ __forceinline__ void tile_states(const float* tile, int n0, int N, in
 // loads and out written with buffer stores; 2: strided with unit channel stride,
 // z and out staged through LDS; 3: as 2, with u staged through the same LDS buffer
 // (its own compile-time case, so that the per-lane u loads of 1 and 2 hold no
-// registers in it). ALN: rows 16-byte aligned (L % 4 == 0, aligned bases), so that
-// rows move in 16-byte pieces; otherwise single floats (SIO 0 only).
+// registers in it). ALN: contiguous rows 16-byte aligned (L % 4 == 0, aligned bases), so
+// that they move in 16-byte pieces; otherwise as single floats (in SIO 2 and 3 that is
+// delta, and u where it is contiguous; what passes through the stage moves in pieces of
+// four channels, whatever L).
 // The row's tail chunk (L % 256 steps) runs in the tile loop as well: its loads and
 // stores check bounds (per lane, by strides, for SIO 1; in the DMA and the stores of
 // the LDS stages of SIO 2 and 3), its B/C positions past the row read zeros, and its
@@ -717,7 +719,7 @@ __device__ __forceinline__ void tile_states(const float* tile, int n0, int N, in
 template <int I, bool REV, int SIO, bool SEG = false, bool ALN = true, bool TAIL = false,
           bool DWBC = !ALN>
 __device__ __forceinline__ void tile_rows(const M1Kern& p, long long blk, int seg = 0) {
-  static_assert(ALN || SIO == 0, "unaligned rows: contiguous z and out only");
+  static_assert(ALN || SIO != 1, "unaligned rows: contiguous or staged z and out");
   constexpr int LPR = 16, RPW = 4;
   using G = Tile<I>;
   constexpr long long CH = G::CH;
@@ -1022,7 +1024,7 @@ __device__ __forceinline__ void fold_rows(const M1Kern& p, long long blk, int se
       float dd[I], uu[I];
       // the segments folded here hold whole chunks: no bounds to check
       load_block<I, REV, ALN>(drow, sb + I, sb, 0.0f, dd, L);
-      if (ALN && p.u_strided) {
+      if (p.u_strided) {
         const long long tlo = REV ? L - sb - I : sb;  // the block's lowest memory step
         load_block_strided<I, REV>(slab_rsrc(p.u + bib * p.us_b, p.u_bytes),
                                    (unsigned)((d * p.us_d + tlo * p.us_t) * 4), p.us_t, uu);
@@ -1101,6 +1103,48 @@ __global__ void __launch_bounds__(256) pad_rows_kernel(const float* __restrict__
   dst[e] = t >= 0 && t < L ? src[r * L + t] : 0.0f;
 }
 
+// B and C of any strides copied to (batch, group, state) rows of pitch ldb floats, each
+// row's data starting `off` floats in and zeros around it, as the tiles read them. One
+// block takes 64 steps of every state of one (batch, group) of B or C, 16 states at a time
+// through LDS: read along the states where those are adjacent (columns of a projection, 64
+// bytes a step), else along the steps, written along the steps. One launch in place of two
+// strided copies and, for rows that are not 16-byte multiples, two padding passes: 20 -> 4
+// us of kernels at B4 L1531 N16, 11 -> 5 at B8 L2048.
+struct PackBC {
+  const float *B, *C;
+  float* dst;  // B's rows, then C's
+  long long bs[4], cs[4];
+  long long L, ldb, off;
+  int groups, N, rows;  // rows: batch * groups * N
+};
+__global__ void __launch_bounds__(256) pack_bc_kernel(PackBC p) {
+  __shared__ float tile[16][65];
+  const bool isc = blockIdx.z != 0;
+  const long long(&s)[4] = isc ? p.cs : p.bs;
+  const int b = blockIdx.y / p.groups, g = blockIdx.y - b * p.groups;
+  const float* src = (isc ? p.C : p.B) + b * s[0] + g * s[1];
+  float* dst = p.dst + ((isc ? (long long)p.rows : 0) + (long long)blockIdx.y * p.N) * p.ldb;
+  const long long e0 = (long long)blockIdx.x * 64;  // first float of the rows' pitch
+  const bool by_state = s[2] == 1;
+  for (int n0 = 0; n0 < p.N; n0 += 16) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = threadIdx.x + 256 * r;
+      const int n = by_state ? i & 15 : i >> 6, e = by_state ? i >> 4 : i & 63;
+      const long long t = e0 + e - p.off;
+      tile[n][e] = n0 + n < p.N && t >= 0 && t < p.L ? src[(n0 + n) * s[2] + t * s[3]] : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = threadIdx.x + 256 * r;
+      const int n = i >> 6, e = i & 63;
+      if (n0 + n < p.N && e0 + e < p.ldb) dst[(n0 + n) * p.ldb + e0 + e] = tile[n][e];
+    }
+    __syncthreads();
+  }
+}
+
 // Block id -> row block for time-major z/out: a 128-byte line of those holds 32
 // channels, two row blocks' worth, so adjacent row blocks go to one XCD (block id
 // mod 8), dispatched back to back, and each line is fetched and written back whole
@@ -1175,18 +1219,21 @@ hipError_t launch_tile(const M1Kern& k, hipStream_t st) {
                        (2 * (size_t)RPB + 1) * k.N + kZerosPad);
   const dim3 grid((unsigned)(segs > 1 ? blocks * segs : blocks)), wg(64 * kWavesPerBlock);
   const bool tail = k.L % Tile<I>::CH != 0;
-  if (segs > 1 && tail)
-    hipLaunchKernelGGL((m1_tile_kernel<I, REV, SIO, true, ALN, true, DWBC>), grid, wg, lds, st,
-                       k);
-  else if (segs > 1)
-    hipLaunchKernelGGL((m1_tile_kernel<I, REV, SIO, true, ALN, false, DWBC>), grid, wg, lds, st,
-                       k);
-  else if (tail)
-    hipLaunchKernelGGL((m1_tile_kernel<I, REV, SIO, false, ALN, true, DWBC>), grid, wg, lds, st,
-                       k);
-  else
-    hipLaunchKernelGGL((m1_tile_kernel<I, REV, SIO, false, ALN, false, DWBC>), grid, wg, lds,
-                       st, k);
+  auto go = [&](auto seg_tag, auto tail_tag) {
+    hipLaunchKernelGGL((m1_tile_kernel<I, REV, SIO, decltype(seg_tag)::value, ALN,
+                                       decltype(tail_tag)::value, DWBC>),
+                       grid, wg, lds, st, k);
+  };
+  using T = std::true_type;
+  using F = std::false_type;
+  if (tail) {
+    if (segs > 1) go(T{}, T{});
+    else go(F{}, T{});
+  } else if (segs > 1) {
+    go(T{}, F{});
+  } else {
+    go(F{}, F{});
+  }
   return hipGetLastError();
 }
 
@@ -1367,17 +1414,48 @@ bool distinct_elements(const long long (&s)[3], const M1Problem& pr) {
   return true;
 }
 
+// Whether z and out can pass through the LDS stage: 16-byte runs of channels in out (and
+// z), and for z a chunk of at least two tiles between issuing the stage and reading it.
+static bool m1_staged_io(const M1Problem& pr) {
+  const long long L = (long long)pr.len, D = (long long)pr.dim;
+  const long long zc[3] = {D * L, L, 1};
+  const long long(&zs)[3] = contiguous_strides(pr.z_stride, pr) ? zc : pr.z_stride;
+  const long long(&os)[3] = contiguous_strides(pr.out_stride, pr) ? zc : pr.out_stride;
+  return os[1] == 1 && os[2] % 4 == 0 && os[0] % 4 == 0 && aligned16(pr.out) &&
+         (!pr.z || (zs[1] == 1 && zs[2] % 4 == 0 && zs[0] % 4 == 0 && aligned16(pr.z) &&
+                    pr.state > kTileStates)) &&
+         M1_TILE_I == 16;
+}
+// Whether delta's rows, and u's where they are contiguous, are whole 16-byte pieces.
+static bool rows_aligned(const M1Problem& pr) {
+  return pr.len % 4 == 0 && aligned16(pr.delta) &&
+         (!contiguous_strides(pr.u_stride, pr) || aligned16(pr.u));
+}
+
 bool m1_strided_supported(const M1Problem& pr, const char** why) {
   auto no = [&](const char* w) {
     if (why) *why = w;
     return false;
   };
-  const bool u_cont = contiguous_strides(pr.u_stride, pr);
-  if (pr.len % 4 != 0 || (u_cont && !aligned16(pr.u)) || !aligned16(pr.delta) ||
-      !aligned16(pr.B) || !aligned16(pr.C))
-    return no("strided z/out need len % 4 == 0 and 16-byte aligned u, delta, B, C");
-  if (pr.dim % 16 != 0 || (pr.dim / pr.groups) % 16 != 0)
-    return no("strided z/out need dim and dim/groups multiples of 16");
+  if (pr.views) {
+    // B and C are packed where they do not lie as the tiles read them; rows that are not
+    // 16-byte pieces need z and out staged (m1_staged_io)
+    if (pr.dim % 16 != 0 || (pr.dim / pr.groups) % 16 != 0)
+      return no("views need dim and dim/groups multiples of 16");
+    for (int i = 0; i < 4; ++i)
+      if (pr.b_stride[i] < 0 || pr.c_stride[i] < 0) return no("negative B/C strides");
+    if (!rows_aligned(pr) && !m1_staged_io(pr))
+      return no("rows that are not 16-byte multiples need z and out with unit channel "
+                "stride, 16-byte steps and more than 8 states");
+    if (pr.batch * pr.groups > 65535) return no("too many batches and groups of B/C views");
+  } else {
+    const bool u_cont = contiguous_strides(pr.u_stride, pr);
+    if (pr.len % 4 != 0 || (u_cont && !aligned16(pr.u)) || !aligned16(pr.delta) ||
+        !aligned16(pr.B) || !aligned16(pr.C))
+      return no("strided z/out need len % 4 == 0 and 16-byte aligned u, delta, B, C");
+    if (pr.dim % 16 != 0 || (pr.dim / pr.groups) % 16 != 0)
+      return no("strided z/out need dim and dim/groups multiples of 16");
+  }
   for (int t = 0; t < 3; ++t) {
     const long long(&s)[3] = t == 2 ? pr.u_stride : t ? pr.out_stride : pr.z_stride;
     if (t == 0 && !pr.z) continue;
@@ -1402,7 +1480,7 @@ hipError_t m1_scan_chunked(const M1Problem& pr, hipStream_t st) {
   const bool vec = pr.len % 4 == 0 && aligned16(pr.u) && aligned16(pr.delta) &&
                    aligned16(pr.B) && aligned16(pr.C) && aligned16(pr.z) && aligned16(pr.out);
   const bool rev = pr.reverse != 0;
-  if (m1_strided_io(pr)) {
+  if (m1_strided_io(pr) || pr.views) {
     if (!m1_strided_supported(pr, nullptr)) return hipErrorInvalidValue;
     const long long L = (long long)pr.len, D = (long long)pr.dim;
     const long long zc[3] = {D * L, L, 1};
@@ -1412,12 +1490,7 @@ hipError_t m1_scan_chunked(const M1Problem& pr, hipStream_t st) {
     k.zs_b = zs[0]; k.zs_d = zs[1]; k.zs_t = zs[2];
     k.os_b = os[0]; k.os_d = os[1]; k.os_t = os[2];
     k.z_bytes = pr.z ? (unsigned)slab_bytes(zs, pr) : 0u;
-    // the LDS stage: 16-byte channel runs of out (and z), and for z a chunk of at
-    // least two tiles between issuing the stage and reading it
-    k.z_dma = os[1] == 1 && os[2] % 4 == 0 && os[0] % 4 == 0 && aligned16(pr.out) &&
-              (!pr.z || (zs[1] == 1 && zs[2] % 4 == 0 && zs[0] % 4 == 0 && aligned16(pr.z) &&
-                         pr.state > kTileStates)) &&
-              M1_TILE_I == 16;
+    k.z_dma = m1_staged_io(pr);
     k.o_bytes = (unsigned)slab_bytes(os, pr);
     if (!contiguous_strides(pr.u_stride, pr)) {
       k.u_strided = 1;
@@ -1426,10 +1499,49 @@ hipError_t m1_scan_chunked(const M1Problem& pr, hipStream_t st) {
       k.u_dma = k.z_dma && k.us_d == 1 && k.us_t % 4 == 0 && k.us_b % 4 == 0 &&
                 aligned16(pr.u);
     }
-    if (k.z_dma)
-      return k.u_dma ? run_tile<3>(k, rev, pr.scratch, pr.scratch_bytes, st)
-                     : run_tile<2>(k, rev, pr.scratch, pr.scratch_bytes, st);
-    return run_tile<1>(k, rev, pr.scratch, pr.scratch_bytes, st);
+    auto scan = [&]() {
+      if (k.z_dma && pr.views && !rows_aligned(pr))
+        return k.u_dma ? run_tile<3, false>(k, rev, pr.scratch, pr.scratch_bytes, st)
+                       : run_tile<2, false>(k, rev, pr.scratch, pr.scratch_bytes, st);
+      if (k.z_dma)
+        return k.u_dma ? run_tile<3>(k, rev, pr.scratch, pr.scratch_bytes, st)
+                       : run_tile<2>(k, rev, pr.scratch, pr.scratch_bytes, st);
+      return run_tile<1>(k, rev, pr.scratch, pr.scratch_bytes, st);
+    };
+    if (!pr.views) return scan();
+    const long long N = (long long)pr.state, G = (long long)pr.groups;
+    auto as_read = [&](const long long (&s)[4], const float* q) {
+      return s[0] == G * N * L && s[1] == N * L && s[2] == L && s[3] == 1 && L % 4 == 0 &&
+             aligned16(q);
+    };
+    if (as_read(pr.b_stride, pr.B) && as_read(pr.c_stride, pr.C)) return scan();
+    PackBC pk{};
+    pk.B = pr.B; pk.C = pr.C;
+    for (int i = 0; i < 4; ++i) {
+      pk.bs[i] = pr.b_stride[i];
+      pk.cs[i] = pr.c_stride[i];
+    }
+    pk.L = L;
+    pk.ldb = (L + 3) & ~3LL;
+    pk.off = rev ? pk.ldb - L : 0;  // reverse chunks end at L: pad in front
+    pk.groups = (int)G; pk.N = (int)N;
+    pk.rows = (int)(pr.batch * G * N);
+    const long long n = pk.rows * pk.ldb;
+    hipError_t e = stream_alloc((void**)&pk.dst, 2 * (size_t)n * sizeof(float), st);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(pack_bc_kernel,
+                       dim3((unsigned)((pk.ldb + 63) / 64), (unsigned)(pr.batch * G), 2),
+                       dim3(256), 0, st, pk);
+    e = hipGetLastError();
+    if (e == hipSuccess) {
+      k.B = pk.dst + pk.off;  // each row's first data float
+      k.C = pk.dst + n + pk.off;
+      k.ldb = pk.ldb;
+      k.bpo = pk.off;
+      e = scan();
+    }
+    const hipError_t fe = stream_free(pk.dst, st);
+    return e != hipSuccess ? e : fe;
   }
   // the tiled path needs every 16-row block inside one batch/group
   const bool tiled = pr.dim % 16 == 0 && (pr.dim / pr.groups) % 16 == 0;

@@ -21,6 +21,10 @@ struct M1Problem {
   // null stride array). Every value is taken as given: a stride of 0 is a broadcast.
   int has_strides;
   long long z_stride[3], out_stride[3], u_stride[3];
+  // Set by the views entry point: B and C by element strides (batch, group, state, step),
+  // and rows of any length and alignment. Needs has_strides.
+  int views;
+  long long b_stride[4], c_stride[4];
   // Caller-provided scratch for the segment maps of the few-rows plan (the
   // allocation-free entry point passes its static device array): when set, nothing
   // is allocated, and the plan is cut to what scratch_bytes holds.

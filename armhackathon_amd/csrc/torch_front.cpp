@@ -43,7 +43,7 @@ namespace {
 
 struct Abi {
   decltype(&arm_scan_selective_scan_f32) scan;
-  decltype(&arm_scan_selective_scan_strided_f32) scan_strided;
+  decltype(&arm_scan_selective_scan_views_f32) scan_views;
   decltype(&arm_scan_selective_state_update_f32) step;
   decltype(&arm_scan_selective_scan_bidirectional_f32) bidir;
   decltype(&arm_scan_mamba3_scan_time_major_f32) m3;
@@ -65,7 +65,7 @@ void bind_one(const py::dict& d, const char* name, F& f) {
 
 void bind(const py::dict& d) {
   bind_one(d, "arm_scan_selective_scan_f32", abi.scan);
-  bind_one(d, "arm_scan_selective_scan_strided_f32", abi.scan_strided);
+  bind_one(d, "arm_scan_selective_scan_views_f32", abi.scan_views);
   bind_one(d, "arm_scan_selective_state_update_f32", abi.step);
   bind_one(d, "arm_scan_selective_scan_bidirectional_f32", abi.bidir);
   bind_one(d, "arm_scan_mamba3_scan_time_major_f32", abi.m3);
@@ -193,9 +193,9 @@ py::object wrap(const Tensor& t) {
 }
 
 // ------------------------------------------------------------------ Mamba-1
-// B, C (batch, state, len) or (batch, groups, state, len)
+// B, C (batch, state, len) or (batch, groups, state, len); contiguous, unless views are read
 Tensor bc4(Call& c, const py::handle& h, int64_t batch, int64_t state, int64_t length,
-           int64_t& groups) {
+           int64_t& groups, bool views) {
   Tensor t = c.get(h);
   if (!c.ok) return {};
   if (t.dim() == 3) t = t.unsqueeze(1);
@@ -205,7 +205,7 @@ Tensor bc4(Call& c, const py::handle& h, int64_t batch, int64_t state, int64_t l
   }
   groups = t.size(1);
   c.ok = t.size(0) == batch && t.size(2) == state && t.size(3) == length;
-  return c.ok ? t.contiguous() : t;
+  return c.ok && !views ? t.contiguous() : t;
 }
 
 struct M1 {
@@ -216,8 +216,8 @@ struct M1 {
   }
 };
 
-// strided: u and z keep their strides
-bool m1_args(Call& c, M1& m, bool strided, const py::handle& u, const py::handle& delta,
+// views: u, z, B and C keep their strides
+bool m1_args(Call& c, M1& m, bool views, const py::handle& u, const py::handle& delta,
              const py::handle& a, const py::handle& b, const py::handle& cc,
              const py::handle& d, const py::handle& z, const py::handle& bias,
              const py::handle& h0) {
@@ -231,14 +231,14 @@ bool m1_args(Call& c, M1& m, bool strided, const py::handle& u, const py::handle
   if (m.a.size(0) != m.dim) return false;
   m.a = m.a.contiguous();
   m.delta = c.rows(delta, {m.batch, m.dim, m.length});
-  m.b = bc4(c, b, m.batch, m.state, m.length, m.groups);
-  m.c = bc4(c, cc, m.batch, m.state, m.length, m.groups);
+  m.b = bc4(c, b, m.batch, m.state, m.length, m.groups, views);
+  m.c = bc4(c, cc, m.batch, m.state, m.length, m.groups, views);
   m.d = c.rows(d, {m.dim}, true);
   m.z = c.get(z, {m.batch, m.dim, m.length}, true);
   m.bias = c.rows(bias, {m.dim}, true);
   m.h0 = c.rows(h0, {m.batch, m.dim, m.state}, true);
   if (!c.ok || m.dim % m.groups) return false;
-  if (!strided) {
+  if (!views) {
     m.u = m.u.contiguous();
     if (m.z.defined()) m.z = m.z.contiguous();
   }
@@ -264,22 +264,28 @@ py::object selective_scan(py::handle u, py::handle delta, py::handle a, py::hand
   return py::make_tuple(wrap(out), wrap(last));
 }
 
-// The conditions of arm_scan_selective_scan_strided_f32 that op.py checks (_strided_ok).
-bool strided_ok(const M1& m) {
-  if (m.length % 4 || m.dim % 16 || (m.dim / m.groups) % 16) return false;
-  if (!aligned(m.delta) || !aligned(m.b) || !aligned(m.c)) return false;
-  if (m.u.is_contiguous() && !aligned(m.u)) return false;
+// Views that arm_scan_selective_scan_views_f32 may read in place: offsets of a batch below
+// 4 GiB, and no broadcast (the custom op materialises those).
+bool views_ok(const M1& m) {
   auto fits = [&](at::IntArrayRef s) {
     return s[0] >= 0 && s[1] >= 0 && s[2] >= 0 &&
            4 * ((m.dim - 1) * s[1] + (m.length - 1) * s[2] + 1) < (int64_t(1) << 32);
   };
   auto view_ok = [&](const Tensor& t) {
     for (int i = 0; i < 3; ++i)
-      if (t.stride(i) == 0 && t.size(i) > 1) return false;  // a broadcast is materialised
+      if (t.stride(i) == 0 && t.size(i) > 1) return false;
     return fits(t.strides());
   };
   const std::array<int64_t, 3> out{m.length * m.dim, 1, m.dim};
-  return fits(out) && view_ok(m.u) && (!m.z.defined() || view_ok(m.z));
+  return m.dim % 16 == 0 && (m.dim / m.groups) % 16 == 0 && fits(out) && view_ok(m.u) &&
+         (!m.z.defined() || view_ok(m.z));
+}
+
+template <int N>
+std::array<long long, N> strides_of(const Tensor& t) {
+  std::array<long long, N> s;
+  for (int i = 0; i < N; ++i) s[i] = t.stride(i);
+  return s;
 }
 
 py::object selective_scan_time_major(py::handle u, py::handle delta, py::handle a,
@@ -288,26 +294,22 @@ py::object selective_scan_time_major(py::handle u, py::handle delta, py::handle 
                                      bool reverse) {
   Call c;
   M1 m;
-  // before any copy: rows the strided kernel cannot take are the custom op's
-  const Tensor rows = c.get(u);
-  if (!c.ok || rows.dim() != 3 || rows.size(2) % 4 || rows.size(1) % 16) return py::none();
-  if (!m1_args(c, m, true, u, delta, a, b, cc, d, z, bias, h0) || !strided_ok(m))
+  if (!m1_args(c, m, true, u, delta, a, b, cc, d, z, bias, h0) || !views_ok(m))
     return py::none();
   RECORD_FUNCTION("arm_scan::selective_scan_time_major", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
   Tensor out = empty(c, {m.batch, m.length, m.dim}).transpose(1, 2);
   Tensor last = empty(c, {m.batch, m.dim, m.state});
   const ArmScanDims dims = m.dims();
-  auto strides = [](const Tensor& t) {
-    return std::array<long long, 3>{t.stride(0), t.stride(1), t.stride(2)};
-  };
-  const auto us = strides(m.u), os = strides(out);
-  const auto zs = m.z.defined() ? strides(m.z) : us;
+  const auto us = strides_of<3>(m.u), os = strides_of<3>(out);
+  const auto zs = m.z.defined() ? strides_of<3>(m.z) : us;
+  const auto bs = strides_of<4>(m.b), cs = strides_of<4>(m.c);
   if (!launch(c.device, [&](void* st) {
-        return abi.scan_strided(&dims, ptr(m.u), m.u.is_contiguous() ? nullptr : us.data(),
-                                ptr(m.delta), ptr(m.a), ptr(m.b), ptr(m.c), ptr(m.d), ptr(m.z),
-                                m.z.defined() ? zs.data() : nullptr, ptr(m.bias), softplus,
-                                reverse, out_ptr(out), os.data(), out_ptr(last), ptr(m.h0), st);
+        return abi.scan_views(&dims, ptr(m.u), m.u.is_contiguous() ? nullptr : us.data(),
+                              ptr(m.delta), ptr(m.a), ptr(m.b), bs.data(), ptr(m.c), cs.data(),
+                              ptr(m.d), ptr(m.z), m.z.defined() ? zs.data() : nullptr,
+                              ptr(m.bias), softplus, reverse, out_ptr(out), os.data(),
+                              out_ptr(last), ptr(m.h0), st);
       }))
     return py::none();
   return py::make_tuple(wrap(out), wrap(last));

@@ -140,6 +140,20 @@ int arm_scan_selective_scan_strided_f32(const ArmScanDims* dims, const float* u,
                                         const long long* out_strides, float* last_state,
                                         const float* h0, void* stream);
 
+/* No reference counterpart: arm_scan_selective_scan_strided_f32 for rows of any length and
+ * alignment, with B and C by element strides too (batch, group, state, step), as a mixer
+ * hands them over (columns of a projection). A null stride array is the contiguous layout.
+ * B and C are packed by one kernel where they do not lie as the scan reads them. Needs dim
+ * and dim / groups multiples of 16; rows that are not 16-byte multiples also need z and out
+ * with unit channel stride, batch and step strides that are multiples of 4, 16-byte aligned
+ * bases and more than 8 states. Anything else returns code 2 before any launch. */
+int arm_scan_selective_scan_views_f32(
+    const ArmScanDims* dims, const float* u, const long long* u_strides, const float* delta,
+    const float* a, const float* b, const long long* b_strides, const float* c,
+    const long long* c_strides, const float* d_skip, const float* z, const long long* z_strides,
+    const float* delta_bias, int delta_softplus, int reverse, float* out,
+    const long long* out_strides, float* last_state, const float* h0, void* stream);
+
 /* No reference counterpart (the reference leaves decoding to upstream,
  * README.md:320-322): one step of the Mamba-1 scan for a generation loop, as
  * transformers' mamba_selective_state_update computes it, in one launch. state
