@@ -1,0 +1,60 @@
+"""The decode steps' 16-byte kernels at the edges of their ranges, against float64: states
+of 1 to 16 lanes a row, blocks whose last rows are missing, B and C by pieces or by strides,
+a window of another width or alignment (the one-thread kernels).
+
+Gate 2e-6 of the largest value: a row's sum of up to 144 products (144 * 2^-24 = 8.6e-6 at
+worst, its square root typical) of states that one 32-bit exponential and two roundings
+make.
+"""
+
+import pytest
+
+from util import case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [4, 8, 12, 16, 64, 128, 144, 6])
+@pytest.mark.parametrize("rows", [(1, 1), (3, 37), (40, 1536)], ids=lambda r: "%dx%d" % r)
+@pytest.mark.parametrize("columns", [False, True])
+def test_state_update(n, rows, columns):
+    import torch
+
+    import armhackathon_amd as arm
+
+    b, d = rows
+    case(f"state update {b}x{d} N {n} columns={columns}")
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    x, dt, z, A = rnd(b, d), rnd(b, d) - 3, rnd(b, d), -torch.rand(d, n, device="cuda") * 4
+    wide = rnd(b, 2 * n + 4)
+    B, C = ((wide[:, 4:4 + n], wide[:, 4 + n:]) if columns
+            else (rnd(b, n + 1)[:, 1:], rnd(n, b).t()))
+    D, bias, h = rnd(d), rnd(d), rnd(b, d, n)
+    f = lambda t: t.double()  # noqa: E731
+    dt64 = torch.nn.functional.softplus(f(dt) + f(bias))
+    want_h = torch.exp(dt64[..., None] * f(A)) * f(h) + (dt64 * f(x))[..., None] * f(B)[:, None]
+    want = ((want_h * f(C)[:, None]).sum(-1) + f(D) * f(x)) * torch.nn.functional.silu(f(z))
+    y = arm.selective_state_update(h, x, dt, A, B, C, D=D, z=z, dt_bias=bias, dt_softplus=True)
+    for got, ref in ((y, want), (h, want_h)):
+        assert ((got.double() - ref).abs().max() / ref.abs().max()).item() < 2e-6
+
+
+@pytest.mark.parametrize("width,offset", [(4, 0), (4, 1), (3, 0), (8, 0)])
+@pytest.mark.parametrize("rows", [(1, 1), (3, 37), (48, 1536)], ids=lambda r: "%dx%d" % r)
+def test_conv_step(width, offset, rows):
+    import torch
+
+    import armhackathon_amd as arm
+
+    b, d = rows
+    case(f"conv step {b}x{d} width {width} offset {offset}")
+    gen = torch.Generator(device="cuda").manual_seed(width + d)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    s = rnd(b * d * width + offset)[offset:].view(b, d, width)
+    w, bias, x = rnd(d, width), rnd(d), rnd(b, 2 * d)[:, d:]
+    win = torch.cat((s[..., 1:], x[..., None]), -1)
+    want = torch.nn.functional.silu((win.double() * w.double()).sum(-1) + bias.double())
+    y = arm.causal_conv1d_update(x, s, w, bias, activation="silu")
+    assert torch.equal(s, win)
+    assert ((y.double() - want).abs().max() / want.abs().max()).item() < 2e-6
