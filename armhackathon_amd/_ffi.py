@@ -181,6 +181,14 @@ def _declare(lib):
                   *([_vp] * 12),         # q k v adt dt trap q_bias k_bias cos sin d_skip z
                   _ci, _ci,              # backend threading
                   _vp, _vp]              # out stream
+    f = lib.arm_scan_mamba3_grid_f32
+    f.restype = _ci
+    f.argtypes = [ctypes.POINTER(ArmMamba3Dims), ctypes.c_size_t, ctypes.c_size_t,
+                  *([_vp] * 9),          # q k v adt dt trap q_bias k_bias angles
+                  ctypes.c_size_t,       # n_angles
+                  _vp, _vp,              # d_skip z
+                  _ci, _ci,              # noncausal merge
+                  _vp, _vp]              # out stream
     f = lib.arm_scan_mamba3_angles_f32
     f.restype = _ci
     f.argtypes = [_vp, _vp,                      # angles dt

@@ -22,7 +22,7 @@ _FUNCTIONS = ("arm_scan_selective_scan_f32", "arm_scan_selective_scan_views_f32"
               "arm_scan_mamba3_scan_strided_f32", "arm_scan_mamba3_noncausal_f32",
               "arm_scan_mamba3_angles_f32", "arm_scan_mamba3_block_frontend_f32",
               "arm_scan_causal_conv1d_f32", "arm_scan_causal_conv1d_update_f32",
-              "arm_scan_ss2d_f32", "arm_scan_thread_scratch")
+              "arm_scan_ss2d_f32", "arm_scan_mamba3_grid_f32", "arm_scan_thread_scratch")
 
 _module = None
 

@@ -18,6 +18,7 @@
 
 #include "../../include/arm_scan_hip.h"
 #include "scan_launch.h"
+#include "m3_grid.h"
 
 namespace {
 
@@ -659,6 +660,82 @@ int arm_scan_mamba3_noncausal_f32(const ArmMamba3Dims* dims, const float* q, con
   return mamba3_call(dims, q, k, v, adt, dt, trap, q_bias, k_bias, cos, sin, d_skip, z,
                      nullptr, nullptr, nullptr, 1, backend, threading, out, nullptr, nullptr,
                      stream, true, nullptr, 0, true);
+}
+
+int arm_scan_mamba3_grid_f32(const ArmMamba3Dims* dims, size_t height, size_t width,
+                             const float* q, const float* k, const float* v, const float* adt,
+                             const float* dt, const float* trap, const float* q_bias,
+                             const float* k_bias, const float* angles, size_t n_angles,
+                             const float* d_skip, const float* z, int noncausal, int merge,
+                             float* out, void* stream) {
+  if (!dims || !q || !k || !v || !adt || !dt || !trap || !q_bias || !k_bias || !angles || !out)
+    return fail(ARM_SCAN_ERR_NULL_POINTER, "a required pointer is null");
+  const ArmMamba3Dims& d = *dims;
+  if (!d.batch || !d.heads || !d.dv || !d.dqk || !height || !width || !d.groups || d.rank != 1)
+    return fail(ARM_SCAN_ERR_INVALID_DIMS, "a dimension is zero, or the rank is not 1");
+  if (merge != 1 && merge != 2)
+    return fail(ARM_SCAN_ERR_BAD_ENUM, "merge must be 1 (sum) or 2 (mean)");
+  if (height > (1u << 15) || width > (1u << 15) || d.len != height * width ||
+      d.batch * d.heads > (1u << 30))
+    return fail(ARM_SCAN_ERR_INVALID_DIMS, "len must be height * width, each up to 32768");
+  if (d.dqk % 2 || n_angles == 0 || n_angles > d.dqk / 2)
+    return fail(ARM_SCAN_ERR_INVALID_DIMS, "n_angles must be 1 .. dqk/2, dqk even");
+  if (!prod_ok({2, d.batch, d.len, d.groups, d.dqk}) ||
+      !prod_ok({2, d.batch, d.len, d.heads, d.dv, 4}) ||
+      !prod_ok({2, d.batch, d.len, d.heads, d.dqk}) || d.heads * d.dv > (1u << 30) ||
+      d.groups * d.dqk > (1u << 30) || d.heads * n_angles > (1u << 30))
+    return fail(ARM_SCAN_ERR_INVALID_DIMS, "dims overflow");
+  // scratch: both orderings of every tensor, cos and sin, and the traversals' outputs, each
+  // section a multiple of 16 bytes
+  const size_t cells = 2 * d.batch * d.len;
+  auto pad = [](size_t n) { return (n + 3) & ~size_t(3); };
+  const size_t n_qk = pad(cells * d.groups * d.dqk), n_v = pad(cells * d.heads * d.dv);
+  const size_t n_g = pad(cells * d.heads), n_a = pad(cells * d.heads * n_angles);
+  const size_t n_cs = pad(cells * d.heads * (d.dqk / 2));
+  const size_t total = 2 * n_qk + (z ? 2 : 1) * n_v + 3 * n_g + n_a + 2 * n_cs +
+                       (noncausal ? 1 : 2) * n_v;
+  hipStream_t st = (hipStream_t)stream;
+  float* base = nullptr;
+  if (hipError_t e = armscan::stream_alloc((void**)&base, total * sizeof(float), st))
+    return hip_fail(e, "grid scratch allocation");
+  float* next = base;
+  auto take = [&](size_t n) {
+    float* r = next;
+    next += n;
+    return r;
+  };
+  float *q2 = take(n_qk), *k2 = take(n_qk), *v2 = take(n_v), *z2 = z ? take(n_v) : nullptr;
+  float *adt2 = take(n_g), *dt2 = take(n_g), *trap2 = take(n_g), *ang2 = take(n_a);
+  float *cos2 = take(n_cs), *sin2 = take(n_cs), *f = take(n_v);
+  float* b = noncausal ? nullptr : take(n_v);
+  const long long B = (long long)d.batch, BH = (long long)(d.batch * d.heads);
+  const int uqk = (int)(d.groups * d.dqk), uv = (int)(d.heads * d.dv);
+  armscan::GridSection secs[8] = {{q, q2, B, uqk, 0},   {k, k2, B, uqk, 0},
+                                  {v, v2, B, uv, 0},    {angles, ang2, B, (int)(d.heads * n_angles), 0},
+                                  {adt, adt2, BH, 1, 0}, {dt, dt2, BH, 1, 0},
+                                  {trap, trap2, BH, 1, 0}};
+  int n = 7;
+  if (z) secs[n++] = {z, z2, B, uv, 0};
+  ArmMamba3Dims d2 = d;
+  d2.batch = 2 * d.batch;
+  int rc = run(armscan::grid_to_views(secs, n, (int)height, (int)width, st), "grid views launch");
+  if (!rc)
+    rc = arm_scan_mamba3_angles_f32(ang2, dt2, d2.batch, d.len, d.heads, n_angles, d.dqk / 2,
+                                    cos2, sin2, stream);
+  if (!rc && noncausal)
+    rc = arm_scan_mamba3_noncausal_f32(&d2, q2, k2, v2, adt2, dt2, trap2, q_bias, k_bias, cos2,
+                                       sin2, d_skip, z2, 0, 0, f, stream);
+  for (int rev = 0; !rc && !noncausal && rev < 2; ++rev)
+    rc = arm_scan_mamba3_scan_time_major_f32(&d2, q2, k2, v2, adt2, dt2, trap2, q_bias, k_bias,
+                                             cos2, sin2, d_skip, z2, nullptr, nullptr, nullptr,
+                                             rev, 0, 0, rev ? b : f, nullptr, nullptr, stream);
+  if (!rc)
+    rc = run(armscan::views_to_grid(out, f, b, (int)d.batch, (int)height, (int)width, uv,
+                                    merge == 1 ? 1.0f : noncausal ? 0.5f : 0.25f, st),
+             "grid merge launch");
+  const hipError_t fe = armscan::stream_free(base, st);
+  if (rc) return rc;
+  return run(fe, "grid scratch free");
 }
 
 int arm_scan_mamba3_angles_f32(const float* angles, const float* dt, size_t batch, size_t len,

@@ -55,6 +55,7 @@ struct Abi {
   decltype(&arm_scan_causal_conv1d_f32) conv;
   decltype(&arm_scan_causal_conv1d_update_f32) conv_step;
   decltype(&arm_scan_ss2d_f32) ss2d;
+  decltype(&arm_scan_mamba3_grid_f32) grid;
   decltype(&arm_scan_thread_scratch) thread_scratch;
 } abi{};
 
@@ -77,6 +78,7 @@ void bind(const py::dict& d) {
   bind_one(d, "arm_scan_causal_conv1d_f32", abi.conv);
   bind_one(d, "arm_scan_causal_conv1d_update_f32", abi.conv_step);
   bind_one(d, "arm_scan_ss2d_f32", abi.ss2d);
+  bind_one(d, "arm_scan_mamba3_grid_f32", abi.grid);
   bind_one(d, "arm_scan_thread_scratch", abi.thread_scratch);
 }
 
@@ -619,6 +621,39 @@ py::object noncausal(py::handle q, py::handle k, py::handle v, py::handle adt, p
   return wrap(out);
 }
 
+// Both orderings of a token grid, scanned and merged: q, k (b, H, W, g, dqk); v, z (b, H, W,
+// h, dv); adt, dt, trap (b, h, H, W); angles (b, H, W, h, r); merge 1 sum, 2 mean.
+py::object grid_mamba3(py::handle q, py::handle k, py::handle v, py::handle adt, py::handle dt,
+                       py::handle trap, py::handle qb, py::handle kb, py::handle ang,
+                       py::handle d, py::handle z, bool noncausal, int merge) {
+  Call c;
+  const Tensor q0 = c.get(q), v0 = c.get(v), a0 = c.get(ang);
+  if (!c.ok || q0.dim() != 5 || v0.dim() != 5 || a0.dim() != 5 || (merge != 1 && merge != 2))
+    return py::none();
+  const int64_t b = q0.size(0), H = q0.size(1), W = q0.size(2), g = q0.size(3),
+                dqk = q0.size(4), h = v0.size(3), dv = v0.size(4), r = a0.size(4);
+  if (dqk % 2 || h % g || r > dqk / 2) return py::none();
+  const Tensor tq = c.rows(q, {b, H, W, g, dqk}), tk = c.rows(k, {b, H, W, g, dqk}),
+               tv = c.rows(v, {b, H, W, h, dv}), tadt = c.rows(adt, {b, h, H, W}),
+               tdt = c.rows(dt, {b, h, H, W}), ttrap = c.rows(trap, {b, h, H, W}),
+               tqb = c.rows(qb, {h, dqk}), tkb = c.rows(kb, {h, dqk}),
+               ta = c.rows(ang, {b, H, W, h, r}), td = c.rows(d, {h}, true),
+               tz = c.rows(z, {b, H, W, h, dv}, true);
+  if (!c.ok) return py::none();
+  RECORD_FUNCTION("arm_scan::mamba3_grid", std::vector<c10::IValue>());
+  c10::DeviceGuard on_device(c.device);
+  Tensor out = empty(c, {b, H, W, h, dv});
+  const ArmMamba3Dims dims{(size_t)b, (size_t)h,       (size_t)dv, (size_t)dqk,
+                           (size_t)(H * W), (size_t)1, (size_t)g};
+  if (!launch(c.device, [&](void* st) {
+        return abi.grid(&dims, H, W, ptr(tq), ptr(tk), ptr(tv), ptr(tadt), ptr(tdt), ptr(ttrap),
+                        ptr(tqb), ptr(tkb), ptr(ta), r, ptr(td), ptr(tz), noncausal, merge,
+                        out_ptr(out), st);
+      }))
+    return py::none();
+  return wrap(out);
+}
+
 // The mixer between its projections: the front-end kernel, then the scan reading z, x and
 // the angles where they lie in proj [z | x | B | C | dd_dt | dd_A | trap | angles].
 py::object mixer_scan(py::handle proj, py::handle dt_bias, py::handle b_norm,
@@ -681,5 +716,6 @@ PYBIND11_MODULE(_torch_front, m) {
   m.def("ss2d", &ss2d);
   m.def("mamba3", &mamba3);
   m.def("noncausal", &noncausal);
+  m.def("grid_mamba3", &grid_mamba3);
   m.def("mixer_scan", &mixer_scan);
 }

@@ -175,6 +175,11 @@ def ss2d_noncausal_mamba3(q, k, v, adt, dt, trap, q_bias, k_bias, angles,
     """
     if merge not in _MERGES:
         raise ValueError(f"merge must be one of {_MERGES}, got {merge!r}")
+    if merge != "none":
+        out = _native("grid_mamba3", q, k, v, adt, dt, trap, q_bias, k_bias, angles, D, z,
+                      True, _ffi.SS2D_MERGES[merge])
+        if out is not None:
+            return out
     if q.dim() != 5:
         raise ValueError(f"q must be (b, H, W, groups, dqk), got {tuple(q.shape)}")
     b, hh, ww = q.shape[:3]

@@ -10,6 +10,8 @@ traversal order, as the reference requires.
 
 import torch
 
+from . import _ffi
+from .op import _native
 from .ss2d import _MERGES, grid_to_views
 
 
@@ -58,6 +60,12 @@ def ss2d_scan_mamba3(q, k, v, adt, dt, trap, q_bias, k_bias, angles, D=None, z=N
     """
     if merge not in _MERGES:
         raise ValueError(f"merge must be one of {_MERGES}, got {merge!r}")
+    if scan_pair is None and merge != "none":
+        # the orderings, the four traversals and the merge in one call of the library
+        out = _native("grid_mamba3", q, k, v, adt, dt, trap, q_bias, k_bias, angles, D, z,
+                      False, _ffi.SS2D_MERGES[merge])
+        if out is not None:
+            return out
     if q.dim() != 5:
         raise ValueError(f"q must be (b, H, W, groups, dqk), got {tuple(q.shape)}")
     b, h, w = q.shape[:3]

@@ -298,6 +298,20 @@ int arm_scan_mamba3_noncausal_f32(const ArmMamba3Dims* dims, const float* q, con
                                   const float* z, int backend, int threading, float* out,
                                   void* stream);
 
+/* No reference counterpart (python/arm_scan/ss2d_mamba3.py and mamba3_noncausal.py compose
+ * it): the Mamba-3 SISO recurrence over a token grid, both orderings of a (height, width)
+ * grid scanned and merged on it. dims.batch grids, dims.len = height * width, rank 1. q, k
+ * (batch, height, width, groups, dqk); v, z (batch, height, width, heads, dv); adt, dt, trap
+ * (batch, heads, height, width); angles (batch, height, width, heads, n_angles), raw; out as
+ * v. noncausal 0: a forward and a backward traversal of each ordering; 1: each ordering's
+ * non-causal sum. merge 1 sum, 2 mean over the traversals (orderings when noncausal). */
+int arm_scan_mamba3_grid_f32(const ArmMamba3Dims* dims, size_t height, size_t width,
+                             const float* q, const float* k, const float* v, const float* adt,
+                             const float* dt, const float* trap, const float* q_bias,
+                             const float* k_bias, const float* angles, size_t n_angles,
+                             const float* d_skip, const float* z, int noncausal, int merge,
+                             float* out, void* stream);
+
 /* No reference counterpart: the RoPE angle pre-pass the reference runs in Python
  * (python/arm_scan/mamba3.py:41-89), as two kernels (the sums of sequence segments,
  * then cos/sin from them). angles (batch, len, heads, n_angles) raw, dt (batch, heads,
