@@ -1339,8 +1339,35 @@ hipError_t m1_noalloc_scratch(float** out, size_t* bytes) {
 }
 
 namespace {
+// Modelled time of a scan of `blocks` row blocks cut into `segs` segments, in microseconds:
+// rounds of 768 resident blocks (three a CU), each as long as its chunks take with one, two
+// or three blocks on a CU (9.1, 11.7 and 15.6 us a chunk at N 16, from B1 to B8 D1536 L2048)
+// and 3 us of start; before them the fold of all segments but the last at 0.75 of that, and
+// 4 us for the second launch. Within 10% of what was measured below, but for several rounds
+// (15%).
+double plan_cost(long long blocks, long long segs, long long nfull, bool tail, int N) {
+  static const double chunk_us[4] = {0.0, 9.1, 11.7, 15.6};
+  auto pass = [&](long long nblk, double chunks, double weight) {
+    double t = 0.0;
+    for (long long left = nblk; left > 0; left -= 768) {
+      const long long per_cu = left >= 768 ? 3 : (left + 255) / 256;
+      t += weight * chunks * chunk_us[per_cu] * N / 16.0 + 3.0;
+    }
+    return t;
+  };
+  const long long len = (nfull + segs - 1) / segs;
+  segs = (nfull + len - 1) / len;  // as many as segments of that length need
+  const long long last = nfull - (segs - 1) * len + (tail ? 1 : 0);
+  const double t = pass(blocks * segs, (double)(len > last ? len : last), 1.0);
+  return segs == 1 ? t : t + pass(blocks * (segs - 1), (double)len, 0.75) + 4.0;
+}
+
 // Rows cut into segments when there are too few to fill the chip: a 16-row block per
-// CU slot, 768 slots (three per CU) resident at once. Sets k.segs / k.seg_chunks and
+// CU slot, 768 slots (three per CU) resident at once, as many segments as the model above
+// finds fastest (whole rows among them). B4 L1531 and L4096 with the convolution 127 -> 112
+// and 287 -> 258 us, B3 L1000 82 -> 70 (whole rows: two blocks a CU already, and no fold
+// pass), B3 L8192 alone 362 -> 311 (eight segments: three even rounds); B1 and B2 L2048 keep
+// eight and four. Sets k.segs / k.seg_chunks and
 // allocates the segment maps on the stream, or, with caller scratch, takes them from
 // it, cutting the plan to fewer segments (down to whole rows, which need no maps)
 // until they fit.
@@ -1352,8 +1379,19 @@ hipError_t plan_segments(M1Kern& k, float* scratch_p, size_t scratch_bytes, hipS
   k.seg_chunks = nfull;
   k.segmap = nullptr;
   if (blocks >= kM1WholeRowBlocks || nfull < 2) return hipSuccess;
-  long long segs = (768 + blocks - 1) / blocks;
-  if (segs > nfull) segs = nfull;
+  long long most = (768 + blocks - 1) / blocks;
+  if (blocks > 192 && most < 8) most = 8;
+  if (most > nfull) most = nfull;
+  long long segs = 1;
+  const bool tail = k.L % (16 * M1_TILE_I) != 0;
+  double best = plan_cost(blocks, 1, nfull, tail, k.N);
+  for (long long s = 2; s <= most; ++s) {
+    const double c = plan_cost(blocks, s, nfull, tail, k.N);
+    if (c < 1.03 * best) {  // near ties: the finer cut, whose blocks end together
+      best = c < best ? c : best;
+      segs = s;
+    }
+  }
   auto map_bytes = [&](long long s) {
     return (size_t)k.rows * (size_t)(s - 1) * (size_t)k.N * 2 * sizeof(float);
   };
