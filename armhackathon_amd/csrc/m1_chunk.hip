@@ -1342,9 +1342,9 @@ namespace {
 // Modelled time of a scan of `blocks` row blocks cut into `segs` segments, in microseconds:
 // rounds of 768 resident blocks (three a CU), each as long as its chunks take with one, two
 // or three blocks on a CU (9.1, 11.7 and 15.6 us a chunk at N 16, from B1 to B8 D1536 L2048)
-// and 3 us of start; before them the fold of all segments but the last at 0.75 of that, and
-// 4 us for the second launch. Within 10% of what was measured below, but for several rounds
-// (15%).
+// and 3 us of start, the last segment's further chunks (the row's tail) on its own blocks;
+// before them the fold of all segments but the last at 0.75 of that, and 4 us for the second
+// launch. Within 10% of what was measured below, but for several rounds (15%).
 double plan_cost(long long blocks, long long segs, long long nfull, bool tail, int N) {
   static const double chunk_us[4] = {0.0, 9.1, 11.7, 15.6};
   auto pass = [&](long long nblk, double chunks, double weight) {
@@ -1358,7 +1358,9 @@ double plan_cost(long long blocks, long long segs, long long nfull, bool tail, i
   const long long len = (nfull + segs - 1) / segs;
   segs = (nfull + len - 1) / len;  // as many as segments of that length need
   const long long last = nfull - (segs - 1) * len + (tail ? 1 : 0);
-  const double t = pass(blocks * segs, (double)(len > last ? len : last), 1.0);
+  const long long alone = (blocks + 255) / 256;  // blocks a CU once only the last one runs
+  const double t = pass(blocks * segs, (double)len, 1.0) +
+                   (last > len ? (last - len) * chunk_us[alone > 3 ? 3 : alone] * N / 16.0 : 0.0);
   return segs == 1 ? t : t + pass(blocks * (segs - 1), (double)len, 0.75) + 4.0;
 }
 
