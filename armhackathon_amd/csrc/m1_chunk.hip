@@ -183,6 +183,49 @@ __device__ __forceinline__ void load_block(const float* __restrict__ row, long l
   }
 }
 
+// The I steps of a lane block of a contiguous row at any float address, by 16-byte loads:
+// global loads need 4-byte alignment only, and as single floats a wave's 16 loads touched 64
+// lines each (B8 D1536 L2047 144 -> 136 us, bidirectional B16 D192 L197 26.1 -> 23.1). In the
+// row's tail (`full` false) a piece that crosses the row's end is read from the row's last
+// four floats and shifted, so that no load branches; steps past the end read 0. Rows of fewer
+// than four steps go by single floats.
+typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
+template <int I, bool REV>
+__device__ __forceinline__ void load_unaligned(const float* __restrict__ row, long long L,
+                                               long long sb, bool full, float (&v)[I]) {
+  const long long mb = REV ? L - sb - I : sb;  // the block's lowest memory step
+  if (!full && L < 4) {                        // wave-uniform
+#pragma unroll
+    for (int i = 0; i < I; ++i) v[i] = sb + i < L ? row[REV ? L - 1 - sb - i : sb + i] : 0.0f;
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < I / 4; ++q) {
+    const long long m = mb + 4 * q;
+    // the four floats read: at m, moved inside the row (down forward, up reverse)
+    const long long at = full ? m : REV ? (m > 0 ? m : 0) : (m < L - 4 ? m : L - 4);
+    const float4_any x = *reinterpret_cast<const float4_any*>(row + at);
+    float w[4] = {x[0], x[1], x[2], x[3]};
+    if (!full) {
+      const long long off = REV ? at - m : m - at;  // by this many; 4 and more: all outside
+      const bool s1 = off == 1, s2 = off == 2, s3 = off == 3, s0 = off == 0;
+      if (REV) {  // w[e] = row[m + e] = x[e - off], 0 below the row
+        w[3] = s0 ? x[3] : s1 ? x[2] : s2 ? x[1] : s3 ? x[0] : 0.0f;
+        w[2] = s0 ? x[2] : s1 ? x[1] : s2 ? x[0] : 0.0f;
+        w[1] = s0 ? x[1] : s1 ? x[0] : 0.0f;
+        w[0] = s0 ? x[0] : 0.0f;
+      } else {  // w[e] = row[m + e] = x[e + off], 0 past the row
+        w[0] = s0 ? x[0] : s1 ? x[1] : s2 ? x[2] : s3 ? x[3] : 0.0f;
+        w[1] = s0 ? x[1] : s1 ? x[2] : s2 ? x[3] : 0.0f;
+        w[2] = s0 ? x[2] : s1 ? x[3] : 0.0f;
+        w[3] = s0 ? x[3] : 0.0f;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[REV ? I - 1 - (4 * q + e) : 4 * q + e] = w[e];
+  }
+}
+
 template <int I, bool REV, bool VEC>
 __device__ __forceinline__ void store_block(float* __restrict__ row, long long Lv, long long sb,
                                             const float (&v)[I], long long L, long long ts = 1) {
@@ -804,12 +847,7 @@ __device__ __forceinline__ void tile_rows(const M1Kern& p, long long blk, int se
         for (int e = 0; e < 4; ++e) v[REV ? I - 1 - (4 * q + e) : 4 * q + e] = w[e];
       }
     } else {
-      // one base per block and immediate offsets: traversal step sbl + i is memory
-      // mb + i (forward) or mb + I-1-i (reverse)
-      const float* base = r + (REV ? L - sbl - I : sbl);
-#pragma unroll
-      for (int i = 0; i < I; ++i)
-        v[i] = full || sbl + i < L ? base[REV ? I - 1 - i : i] : 0.0f;
+      load_unaligned<I, REV>(r, L, sbl, full, v);
     }
   };
 
@@ -1023,13 +1061,16 @@ __device__ __forceinline__ void fold_rows(const M1Kern& p, long long blk, int se
     {
       float dd[I], uu[I];
       // the segments folded here hold whole chunks: no bounds to check
-      load_block<I, REV, ALN>(drow, sb + I, sb, 0.0f, dd, L);
+      if constexpr (ALN) load_block<I, REV, true>(drow, sb + I, sb, 0.0f, dd, L);
+      else load_unaligned<I, REV>(drow, L, sb, true, dd);
       if (p.u_strided) {
         const long long tlo = REV ? L - sb - I : sb;  // the block's lowest memory step
         load_block_strided<I, REV>(slab_rsrc(p.u + bib * p.us_b, p.u_bytes),
                                    (unsigned)((d * p.us_d + tlo * p.us_t) * 4), p.us_t, uu);
+      } else if constexpr (ALN) {
+        load_block<I, REV, true>(urow, sb + I, sb, 0.0f, uu, L);
       } else {
-        load_block<I, REV, ALN>(urow, sb + I, sb, 0.0f, uu, L);
+        load_unaligned<I, REV>(urow, L, sb, true, uu);
       }
 #pragma unroll
       for (int i = 0; i < I; ++i) {
