@@ -748,9 +748,9 @@ __device__ __forceinline__ void tile_states(const float* tile, int n0, int N, in
 // z and out staged through LDS; 3: as 2, with u staged through the same LDS buffer
 // (its own compile-time case, so that the per-lane u loads of 1 and 2 hold no
 // registers in it). ALN: contiguous rows 16-byte aligned (L % 4 == 0, aligned bases), so
-// that they move in 16-byte pieces; otherwise as single floats (in SIO 2 and 3 that is
-// delta, and u where it is contiguous; what passes through the stage moves in pieces of
-// four channels, whatever L).
+// that they move in 16-byte pieces; otherwise by load_unaligned and the out stage (in SIO 2
+// and 3 that is delta, and u where it is contiguous; what passes through the stage moves in
+// pieces of four channels, whatever L).
 // The row's tail chunk (L % 256 steps) runs in the tile loop as well: its loads and
 // stores check bounds (per lane, by strides, for SIO 1; in the DMA and the stores of
 // the LDS stages of SIO 2 and 3), its B/C positions past the row read zeros, and its
@@ -1628,7 +1628,8 @@ hipError_t m1_scan_chunked(const M1Problem& pr, hipStream_t st) {
   const bool tiled = pr.dim % 16 == 0 && (pr.dim / pr.groups) % 16 == 0;
   if (!tiled) return launch_dir<16, 16>(k, rev, vec, st);
   if (vec) return run_tile<0, true>(k, rev, pr.scratch, pr.scratch_bytes, st);
-  // Rows that are not 16-byte multiples: u, delta, z and out move as single floats.
+  // Rows that are not 16-byte multiples: u, delta and z by load_unaligned, out as single
+  // floats through LDS.
   // B and C (shared by every channel, a few MB) are copied to a row pitch rounded up
   // to 4 so that the tiles still fill by 16-byte DMA (B8 D1536 L2050: 209 -> 187 us
   // with 16-byte DMA). The allocation-free entry, which owns no memory for the copy,
