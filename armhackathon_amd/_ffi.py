@@ -103,19 +103,6 @@ def _declare(lib):
                   _vp, _vp,              # out out_strides
                   _vp, _vp,              # last_state h0
                   _vp]                   # stream
-    f = lib.arm_scan_selective_scan_views_f32
-    f.restype = _ci
-    f.argtypes = [ctypes.POINTER(ArmScanDims),
-                  _vp, _vp, _vp, _vp,    # u u_strides delta a
-                  _vp, _vp, _vp, _vp,    # b b_strides c c_strides
-                  _vp, _vp, _vp, _vp,    # d_skip z z_strides delta_bias
-                  _ci, _ci,              # delta_softplus reverse
-                  _vp, _vp,              # out out_strides
-                  _vp, _vp,              # last_state h0
-                  _vp]                   # stream
-    f = lib.arm_scan_thread_scratch
-    f.restype = None
-    f.argtypes = [_vp, _vp]              # alloc ctx
     f = lib.arm_scan_selective_state_update_f32
     f.restype = _ci
     f.argtypes = [*([ctypes.c_size_t] * 3),      # batch dim state_dim
@@ -181,14 +168,6 @@ def _declare(lib):
                   *([_vp] * 12),         # q k v adt dt trap q_bias k_bias cos sin d_skip z
                   _ci, _ci,              # backend threading
                   _vp, _vp]              # out stream
-    f = lib.arm_scan_mamba3_grid_f32
-    f.restype = _ci
-    f.argtypes = [ctypes.POINTER(ArmMamba3Dims), ctypes.c_size_t, ctypes.c_size_t,
-                  *([_vp] * 9),          # q k v adt dt trap q_bias k_bias angles
-                  ctypes.c_size_t,       # n_angles
-                  _vp, _vp,              # d_skip z
-                  _ci, _ci,              # noncausal merge
-                  _vp, _vp]              # out stream
     f = lib.arm_scan_mamba3_angles_f32
     f.restype = _ci
     f.argtypes = [_vp, _vp,                      # angles dt
@@ -201,6 +180,32 @@ def _declare(lib):
                   _ci, _ci,              # delta_softplus merge
                   _vp, _vp,              # out last_states
                   _vp]                   # stream
+    # called by the native front-end alone (_front.py); a library of the same ABI version
+    # without them serves everything else
+    if hasattr(lib, "arm_scan_selective_scan_views_f32"):
+        f = lib.arm_scan_selective_scan_views_f32
+        f.restype = _ci
+        f.argtypes = [ctypes.POINTER(ArmScanDims),
+                      _vp, _vp, _vp, _vp,    # u u_strides delta a
+                      _vp, _vp, _vp, _vp,    # b b_strides c c_strides
+                      _vp, _vp, _vp, _vp,    # d_skip z z_strides delta_bias
+                      _ci, _ci,              # delta_softplus reverse
+                      _vp, _vp,              # out out_strides
+                      _vp, _vp,              # last_state h0
+                      _vp]                   # stream
+    if hasattr(lib, "arm_scan_thread_scratch"):
+        f = lib.arm_scan_thread_scratch
+        f.restype = None
+        f.argtypes = [_vp, _vp]              # alloc ctx
+    if hasattr(lib, "arm_scan_mamba3_grid_f32"):
+        f = lib.arm_scan_mamba3_grid_f32
+        f.restype = _ci
+        f.argtypes = [ctypes.POINTER(ArmMamba3Dims), ctypes.c_size_t, ctypes.c_size_t,
+                      *([_vp] * 9),          # q k v adt dt trap q_bias k_bias angles
+                      ctypes.c_size_t,       # n_angles
+                      _vp, _vp,              # d_skip z
+                      _ci, _ci,              # noncausal merge
+                      _vp, _vp]              # out stream
 
 
 def load():
