@@ -30,6 +30,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
+#include <torch/version.h>
 
 #include <array>
 #include <initializer_list>
@@ -706,6 +707,7 @@ py::object mixer_scan(py::handle proj, py::handle dt_bias, py::handle b_norm,
 }  // namespace
 
 PYBIND11_MODULE(_torch_front, m) {
+  m.attr("torch_version") = TORCH_VERSION;
   m.def("bind", &bind);
   m.def("selective_scan", &selective_scan);
   m.def("selective_scan_time_major", &selective_scan_time_major);

@@ -1,7 +1,13 @@
-"""A library of the same ABI version without the functions that only the native eager
-front-end calls is declared and used, as it was before they were added."""
+"""Where the native eager front-end cannot be had, the public calls take the custom ops, as
+they did before it existed: no error of the loader's reaches the caller."""
 
-from armhackathon_amd import _ffi
+import warnings
+
+import pytest
+
+from armhackathon_amd import _ffi, _front
+
+torch = pytest.importorskip("torch")
 
 
 class Without:
@@ -22,3 +28,31 @@ class Without:
 
 def test_older_library_is_declared():
     _ffi._declare(Without(_ffi.load()))
+
+
+@pytest.mark.parametrize("why", ["missing", "not loadable", "older library", "other torch"])
+def test_absent_front_end_leaves_the_custom_op(why, tmp_path, monkeypatch):
+    import armhackathon_amd as arm_scan
+
+    _ffi.load()
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(_front, "_module", None)
+    monkeypatch.setattr(_front, "_absent", False, raising=False)
+    if why == "missing":
+        monkeypatch.setattr(_front, "_PATH", tmp_path / "none.so")
+    elif why == "not loadable":
+        bad = tmp_path / "_torch_front.so"
+        bad.write_bytes(b"not a library")
+        monkeypatch.setattr(_front, "_PATH", bad)
+    elif why == "older library":
+        monkeypatch.setattr(_ffi, "_lib", Without(_ffi.load()))
+    else:
+        monkeypatch.setattr(torch, "__version__", "1.0.0+other")
+    u = torch.zeros(1, 2, 8)
+    bc = torch.zeros(1, 4, 8)
+    with pytest.warns(RuntimeWarning, match="front-end is not in use"):
+        with pytest.raises(ValueError, match="device tensors"):  # the custom op's refusal
+            arm_scan.selective_scan(u, u, torch.zeros(2, 4), bc, bc)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")  # told once
+        assert _front.front() is None
