@@ -79,6 +79,7 @@ _lib = None
 _lib_path = None
 
 _vp, _ci = ctypes.c_void_p, ctypes.c_int
+SCRATCH_ALLOC = ctypes.CFUNCTYPE(_vp, _vp, ctypes.c_size_t)  # arm_scan_thread_scratch's alloc
 
 
 def _declare(lib):

@@ -141,7 +141,7 @@ namespace armscan {
 // given since it was set. A stream-ordered allocation and its free cost the host 9 us of a
 // call, 14 with the kernels between them, where torch's caching allocator takes 1.
 struct ThreadScratch {
-  static constexpr int kMost = 8;  // a call takes at most three
+  static constexpr int kMost = 8;  // a call takes at most four (a causal Mamba-3 grid)
   void* (*alloc)(void*, size_t) = nullptr;
   void* ctx = nullptr;
   void* given[kMost] = {};
@@ -162,20 +162,23 @@ void thread_scratch(void* (*alloc)(void*, size_t), void* ctx) {
 // steady stream of calls allocates from memory already mapped; the device's default
 // pool, which the caller or torch may use, keeps its own settings. Where a pool cannot
 // be created, the scratch comes from the default pool as it is.
+//
+// A stream under capture takes its scratch from the thread's own source or not at all: from
+// the pool the graph would hold an allocation and a free for every block of every call, and
+// the replay of one such graph of several calls ended in a memory fault.
 hipError_t stream_alloc(void** p, size_t bytes, hipStream_t st) {
   if (t_scratch.alloc != nullptr && t_scratch.n < ThreadScratch::kMost) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
-      (void)hipGetLastError();  // e.g. the null stream beside a capture: the pool, as ever
-      status = hipStreamCaptureStatusActive;
-    }
-    if (status == hipStreamCaptureStatusNone) {
-      *p = t_scratch.alloc(t_scratch.ctx, bytes);
-      if (*p == nullptr) return hipErrorOutOfMemory;
-      t_scratch.given[t_scratch.n++] = *p;
-      return hipSuccess;
-    }
+    *p = t_scratch.alloc(t_scratch.ctx, bytes);
+    if (*p == nullptr) return hipErrorOutOfMemory;
+    t_scratch.given[t_scratch.n++] = *p;
+    return hipSuccess;
   }
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+    (void)hipGetLastError();  // the null stream beside a capture: not captured itself
+    status = hipStreamCaptureStatusNone;
+  }
+  if (status != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
   constexpr int kMaxDevices = 64;
   static std::atomic<hipMemPool_t> pools[kMaxDevices] = {};
   static std::atomic<bool> no_pool[kMaxDevices] = {};

@@ -184,7 +184,7 @@ bool m3_chunk_supported(const M3Problem& p);
 hipError_t m3_scan_chunked(const M3Problem& p, hipStream_t st);
 
 // Stream-ordered scratch: from the calling thread's own source (arm_scan_thread_scratch)
-// where it set one and st is not being captured, else from the library's pool.
+// where it set one, else from the library's pool (refused while st is being captured).
 hipError_t stream_alloc(void** p, size_t bytes, hipStream_t st);
 // Gives it back after what has been enqueued on st.
 hipError_t stream_free(void* p, hipStream_t st);

@@ -29,7 +29,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _ffi
-from .op import _CALLS, _c, _device_of, _native, _ptr, _stream
+from .op import _CALLS, _c, _device_of, _native, _on, _ptr, _stream
 
 
 def angles_to_cos_sin(angles: torch.Tensor, dt: torch.Tensor,
@@ -54,7 +54,7 @@ def angles_to_cos_sin(angles: torch.Tensor, dt: torch.Tensor,
         a, d = angles.contiguous(), dt.contiguous()
         cos = torch.empty((b, length, h, half), dtype=torch.float32, device=a.device)
         sin = torch.empty_like(cos)
-        with torch.cuda.device(a.device):
+        with _on(a.device):
             _ffi.angles_raw(a.data_ptr(), d.data_ptr(), b, length, h, r, half, cos.data_ptr(),
                             sin.data_ptr(), stream=_stream(a.device))
         return cos, sin
@@ -88,7 +88,7 @@ def _run(q, k, v, adt, dt, trap, q_bias, k_bias, cos, sin, d_skip, z, reverse, p
         if want_state else None
     last_bx = torch.empty((b, h, dqk), dtype=torch.float32, device=dev) \
         if (want_state and not mimo) else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.mamba3_raw(
             dims,
             [q.data_ptr(), k.data_ptr(), v.data_ptr(), adt.data_ptr(), dt.data_ptr(),
@@ -126,7 +126,7 @@ def _run_angles(q, k, v, adt, dt, trap, q_bias, k_bias, angles, d_skip, z, psi, 
         if want_state else None
     last_bx = torch.empty((b, h, dqk), dtype=torch.float32, device=dev) \
         if (want_state and not mimo) else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.mamba3_angles_raw(
             dims,
             [q.data_ptr(), k.data_ptr(), v.data_ptr(), adt.data_ptr(), dt.data_ptr(),
@@ -210,7 +210,7 @@ def _run_strided(q, k, v, adt, dt, trap, q_bias, k_bias, angles, d_skip, z, psi,
     h, dv = v.shape[2], v.shape[3]
     dims = _ffi.ArmMamba3Dims(b, h, dv, dqk, length, rank, groups)
     out = torch.empty((b, length, h, dv), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.mamba3_strided_raw(
             dims,
             [q.data_ptr(), k.data_ptr(), v.data_ptr(), adt.data_ptr(), dt.data_ptr(),

@@ -32,7 +32,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _ffi
-from .op import _CALLS, _device_of, _native, _stream
+from .op import _CALLS, _device_of, _native, _on, _stream
 
 
 def heavy_tail_activation(x: torch.Tensor) -> torch.Tensor:
@@ -77,7 +77,7 @@ def _mixer_scan(proj, dt_bias, b_norm, c_norm, b_bias, c_bias, d_skip, psi, zeta
     col_ang = 2 * d_inner + 2 * rank * groups * d_state + 3 * heads
     out = torch.empty((b, length, heads, headdim), **f32)
     base, es = proj.data_ptr(), proj.element_size()
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _stream(dev)
         _ffi.block_frontend_raw(
             base, b, length, row, heads, headdim, d_state, rank, groups, n_angles,

@@ -27,7 +27,7 @@ import torch
 
 from . import _ffi
 from .mamba3 import _check_shapes, _cos_sin
-from .op import _CALLS, _c, _device_of, _native, _ptr, _stream
+from .op import _CALLS, _c, _device_of, _native, _on, _ptr, _stream
 from .ss2d import _MERGES, grid_to_views
 from .ss2d_mamba3 import _check_grid, grid_to_views_time_major, views_to_grid_time_major
 
@@ -38,7 +38,7 @@ def _run_noncausal(q, k, v, adt, dt, trap, q_bias, k_bias, cos, sin, d_skip, z):
     h, dv = v.shape[2], v.shape[3]
     dims = _ffi.ArmMamba3Dims(b, h, dv, dqk, length, 1, groups)
     out = torch.empty((b, length, h, dv), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.mamba3_noncausal_raw(
             dims,
             [q.data_ptr(), k.data_ptr(), v.data_ptr(), adt.data_ptr(), dt.data_ptr(),

@@ -17,6 +17,7 @@ checks and the same kernels, a third of the host time. Everything else, and ever
 is the custom op's.
 """
 
+import ctypes
 from typing import Optional, Tuple
 
 import torch
@@ -53,6 +54,36 @@ def _device_of(*tensors):
 
 def _stream(dev):
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+class _on(torch.cuda.device):
+    """The device of a library call made through ctypes. While the current stream is being
+    captured the call's scratch comes from torch's allocator, whose blocks belong to the
+    graph then; the library's own pool does not serve a capture."""
+
+    def __enter__(self):
+        super().__enter__()
+        self._held = None
+        lib = _ffi.load()
+        if torch.cuda.is_current_stream_capturing() and hasattr(lib, "arm_scan_thread_scratch"):
+            self._held = []
+
+            def alloc(_, nbytes):
+                try:
+                    t = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+                except RuntimeError:  # out of memory: the library reports it
+                    return None
+                self._held.append(t)
+                return t.data_ptr()
+
+            self._alloc = _ffi.SCRATCH_ALLOC(alloc)
+            lib.arm_scan_thread_scratch(ctypes.cast(self._alloc, ctypes.c_void_p), None)
+
+    def __exit__(self, *exc):
+        if self._held is not None:
+            _ffi.load().arm_scan_thread_scratch(None, None)
+            self._held = self._alloc = None
+        return super().__exit__(*exc)
 
 
 def _native(name, *args):
@@ -111,7 +142,7 @@ def _selective_scan_op(
     out = torch.empty_like(u)
     last_state = u.new_empty((batch, dim, state))
     dims = _ffi.ArmScanDims(batch, dim, length, state, groups)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.scan_raw(dims, u.data_ptr(), delta.data_ptr(), a.data_ptr(), b.data_ptr(),
                       c.data_ptr(), _ptr(d_skip), _ptr(z), _ptr(delta_bias), delta_softplus,
                       "auto", "auto", out.data_ptr(), last_state.data_ptr(), ptr_h0=_ptr(h0),
@@ -201,7 +232,7 @@ def _selective_scan_tm_op(
     out = u.new_empty((batch, length, dim)).transpose(1, 2)
     last_state = u.new_empty((batch, dim, state))
     dims = _ffi.ArmScanDims(batch, dim, length, state, groups)
-    with torch.cuda.device(dev):
+    with _on(dev):
         if _strided_ok(u, delta, b, c, z, dim, length, groups):
             _ffi.scan_strided_raw(dims, u.data_ptr(), delta.data_ptr(), a.data_ptr(),
                                   b.data_ptr(), c.data_ptr(), _ptr(d_skip), _ptr(z),
@@ -291,7 +322,7 @@ def _state_update_op(
     if not state.is_contiguous():
         raise ValueError("state must be contiguous (it is updated in place)")
     out = x.new_empty((batch, dim))
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.state_update_raw(batch, dim, n, state.data_ptr(), x.data_ptr(), x.stride(),
                               dt.data_ptr(), dt.stride(), a.data_ptr(), b.data_ptr(), b.stride(),
                               c.data_ptr(), c.stride(), _ptr(d_skip), _ptr(z),
@@ -340,7 +371,7 @@ def _selective_scan_bidir_op(
     out_fwd = torch.empty_like(u)
     out_bwd = torch.empty_like(u)
     dims = _ffi.ArmScanDims(batch, dim, length, state, groups)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.scan_bidir_raw(dims, u.data_ptr(), delta.data_ptr(), a.data_ptr(), b.data_ptr(),
                             c.data_ptr(), _ptr(d_skip), _ptr(z), _ptr(delta_bias),
                             delta_softplus, "auto", "auto", out_fwd.data_ptr(),
@@ -392,7 +423,7 @@ def selective_scan_bidirectional_with_state(u, delta, A, B, C, D=None, z=None,
     of, ob = torch.empty_like(u), torch.empty_like(u)
     lf, lb = u.new_empty((batch, dim, state)), u.new_empty((batch, dim, state))
     dims = _ffi.ArmScanDims(batch, dim, length, state, groups)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.scan_bidir_raw(dims, u.data_ptr(), delta.data_ptr(), A.data_ptr(), B.data_ptr(),
                             C.data_ptr(), _ptr(D), _ptr(z), _ptr(delta_bias), delta_softplus,
                             "auto", "auto", of.data_ptr(), ob.data_ptr(), lf.data_ptr(),
@@ -411,7 +442,7 @@ def _causal_conv1d_op(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
                           device=dev).transpose(1, 2)
     else:
         out = torch.empty((batch, dim, length), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.causal_conv1d_raw(batch, dim, length, weight.shape[1], x.data_ptr(), x.stride(),
                                weight.data_ptr(), _ptr(bias), silu, out.data_ptr(),
                                stream=_stream(dev), time_major=time_major)
@@ -456,7 +487,7 @@ def _causal_conv1d_update_op(x: torch.Tensor, conv_state: torch.Tensor, weight: 
     dev = _device_of(x, conv_state, weight, bias)
     batch, dim = x.shape
     out = torch.empty((batch, dim), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.causal_conv1d_update_raw(batch, dim, weight.shape[1], x.data_ptr(), x.stride(),
                                       conv_state.data_ptr(), weight.data_ptr(), _ptr(bias),
                                       silu, out.data_ptr(), stream=_stream(dev))

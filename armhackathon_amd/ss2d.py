@@ -17,7 +17,7 @@ view-based composition over the bidirectional scan instead.
 import torch
 
 from . import _ffi
-from .op import _CALLS, _c, _device_of, _native, _ptr, _stream
+from .op import _CALLS, _c, _device_of, _native, _on, _ptr, _stream
 
 _MERGES = ("sum", "mean", "none")
 
@@ -138,7 +138,7 @@ def ss2d_scan(u, delta, A, B, C, D=None, delta_bias=None, delta_softplus=True,
     last = torch.empty((4, b, d, n), dtype=torch.float32, device=dev) \
         if return_last_state else None
     dims = _ffi.ArmSS2DDims(b, d, h, w, n)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _ffi.ss2d_raw(dims, u.data_ptr(), delta.data_ptr(), A.data_ptr(), B.data_ptr(),
                       C.data_ptr(), _ptr(D), _ptr(z), _ptr(delta_bias), delta_softplus, merge,
                       out.data_ptr(), _ptr(last), stream=_stream(dev))

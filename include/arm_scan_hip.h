@@ -343,9 +343,11 @@ int arm_scan_ss2d_f32(const ArmSS2DDims* dims, const float* u, const float* delt
  * `alloc(ctx, bytes)` returns device memory of the current device, 16-byte aligned, which
  * the caller keeps until the call has returned and after that gives back in the order of
  * the call's stream (NULL: out of memory, the call fails with code 6). Null `alloc`: the
- * library's stream-ordered pool, as for every thread that never set one; calls on a stream
- * that is being captured take the pool in any case. A caller sets it around a call:
- * the setting is this thread's alone. */
+ * library's stream-ordered pool, as for every thread that never set one. The pool does not
+ * serve a stream that is being captured: there a call that needs scratch takes it from
+ * `alloc`, whose memory must then live as long as the graph, or fails with code 6
+ * (arm_scan_selective_scan_noalloc_f32 needs none). A caller sets it around a call: the
+ * setting is this thread's alone. */
 void arm_scan_thread_scratch(void* (*alloc)(void* ctx, size_t bytes), void* ctx);
 
 /* Human-readable reason for the last nonzero code returned on this thread. */

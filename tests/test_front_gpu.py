@@ -197,8 +197,9 @@ def test_state_version_counts():
 
 
 def test_scratch_during_capture():
-    """Captured with torch's graphs, a call takes its scratch from the library's pool; each
-    replay equals the eager result, with eager calls between that reuse torch's blocks."""
+    """Captured with torch's graphs, a call takes its scratch from the graph's own blocks of
+    torch's allocator; each replay equals the eager result, with eager calls between that
+    reuse torch's other blocks."""
     import torch
 
     import armhackathon_amd as arm
@@ -224,3 +225,69 @@ def test_scratch_during_capture():
         assert torch.equal(out, want)
         torch.full((4096, 256), float(i), device="cuda")
         assert torch.equal(run(), want)
+
+
+def _node_types(graph):
+    import ctypes
+
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    vp = ctypes.c_void_p
+    hip.hipGraphGetNodes.argtypes = [vp, vp, ctypes.POINTER(ctypes.c_size_t)]
+    hip.hipGraphNodeGetType.argtypes = [vp, ctypes.POINTER(ctypes.c_int)]
+    count = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0
+    nodes = (vp * max(count.value, 1))()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(count)) == 0
+    kinds = set()
+    for i in range(count.value):
+        kind = ctypes.c_int(-1)
+        assert hip.hipGraphNodeGetType(nodes[i], ctypes.byref(kind)) == 0
+        kinds.add(kind.value)
+    return kinds
+
+
+@pytest.mark.parametrize("native", [True, False], ids=["front-end", "custom op"])
+def test_capture_records_kernels_only(native, monkeypatch):
+    """No call leaves an allocation or a free in a captured graph, whichever way it goes: its
+    scratch is torch's. The graphs are looked at and not launched."""
+    import torch
+
+    from armhackathon_amd import op
+
+    calls = _calls()
+    names = ("m3_cos", "m3_angles_odd", "m3_carry", "mimo_angles", "ss2d", "noncausal", "bidir",
+             "scan_views")
+    for name in names:
+        calls[name]()
+    if not native:
+        monkeypatch.setattr(op, "front", lambda: None)
+    for name in names:
+        case(f"capture, {'front-end' if native else 'custom op'}: {name}")
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            out = calls[name]()
+        assert _node_types(g.raw_cuda_graph()) == {0}, name  # hipGraphNodeTypeKernel
+        del out, g
+
+
+def test_capture_without_a_source_of_scratch_is_refused():
+    """Through the C ABI alone a captured call that needs scratch fails, and nothing of it is
+    recorded."""
+    import ctypes
+
+    import torch
+
+    from armhackathon_amd import _ffi
+
+    b, d, n, L = 1, 32, 16, 1024
+    u, dl = _rand(b, d, L), _rand(b, d, L, seed=1)
+    A, B, out = -torch.rand(d, n, device="cuda"), _rand(b, n, L, seed=2), torch.empty_like(u)
+    case("capture through the C ABI")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        rc = _ffi.load().arm_scan_selective_scan_f32(
+            ctypes.byref(_ffi.ArmScanDims(b, d, L, n, 1)), u.data_ptr(), dl.data_ptr(),
+            A.data_ptr(), B.data_ptr(), B.data_ptr(), None, None, None, 1, 0, 0, 0,
+            out.data_ptr(), None, None, torch.cuda.current_stream().cuda_stream)
+    assert rc == 6 and _node_types(g.raw_cuda_graph()) == set()
