@@ -140,17 +140,20 @@ struct Call {
     ok = t.device() == device;
     return t;
   }
-  // with a shape to match, and contiguous (the wrappers' own copy)
+  // with a shape to match
   Tensor get(const py::handle& h, Shape shape, bool optional = false) {
     Tensor t = get(h, optional);
     if (ok && t.defined()) ok = t.sizes().equals(at::IntArrayRef(shape));
     return t;
   }
-  Tensor rows(const py::handle& h, Shape shape, bool optional = false) {
-    Tensor t = get(h, shape, optional);
-    return ok && t.defined() ? t.contiguous() : t;
-  }
 };
+
+// The wrappers' own contiguous copies, made once nothing about the call is left to refuse: a
+// call that goes on to the custom op, which makes them too, has paid for none here.
+void lay(std::initializer_list<Tensor*> ts) {
+  for (Tensor* t : ts)
+    if (t->defined()) *t = t->contiguous();
+}
 
 const float* ptr(const Tensor& t) { return t.defined() ? t.const_data_ptr<float>() : nullptr; }
 float* out_ptr(Tensor& t) { return t.defined() ? t.mutable_data_ptr<float>() : nullptr; }
@@ -196,9 +199,9 @@ py::object wrap(const Tensor& t) {
 }
 
 // ------------------------------------------------------------------ Mamba-1
-// B, C (batch, state, len) or (batch, groups, state, len); contiguous, unless views are read
+// B, C (batch, state, len) or (batch, groups, state, len)
 Tensor bc4(Call& c, const py::handle& h, int64_t batch, int64_t state, int64_t length,
-           int64_t& groups, bool views) {
+           int64_t& groups) {
   Tensor t = c.get(h);
   if (!c.ok) return {};
   if (t.dim() == 3) t = t.unsqueeze(1);
@@ -208,7 +211,7 @@ Tensor bc4(Call& c, const py::handle& h, int64_t batch, int64_t state, int64_t l
   }
   groups = t.size(1);
   c.ok = t.size(0) == batch && t.size(2) == state && t.size(3) == length;
-  return c.ok && !views ? t.contiguous() : t;
+  return t;
 }
 
 struct M1 {
@@ -219,8 +222,8 @@ struct M1 {
   }
 };
 
-// views: u, z, B and C keep their strides
-bool m1_args(Call& c, M1& m, bool views, const py::handle& u, const py::handle& delta,
+// Checked, as they lie: m1_lay makes the rows contiguous.
+bool m1_args(Call& c, M1& m, const py::handle& u, const py::handle& delta,
              const py::handle& a, const py::handle& b, const py::handle& cc,
              const py::handle& d, const py::handle& z, const py::handle& bias,
              const py::handle& h0) {
@@ -232,20 +235,19 @@ bool m1_args(Call& c, M1& m, bool views, const py::handle& u, const py::handle& 
   m.length = m.u.size(2);
   m.state = m.a.size(1);
   if (m.a.size(0) != m.dim) return false;
-  m.a = m.a.contiguous();
-  m.delta = c.rows(delta, {m.batch, m.dim, m.length});
-  m.b = bc4(c, b, m.batch, m.state, m.length, m.groups, views);
-  m.c = bc4(c, cc, m.batch, m.state, m.length, m.groups, views);
-  m.d = c.rows(d, {m.dim}, true);
+  m.delta = c.get(delta, {m.batch, m.dim, m.length});
+  m.b = bc4(c, b, m.batch, m.state, m.length, m.groups);
+  m.c = bc4(c, cc, m.batch, m.state, m.length, m.groups);
+  m.d = c.get(d, {m.dim}, true);
   m.z = c.get(z, {m.batch, m.dim, m.length}, true);
-  m.bias = c.rows(bias, {m.dim}, true);
-  m.h0 = c.rows(h0, {m.batch, m.dim, m.state}, true);
-  if (!c.ok || m.dim % m.groups) return false;
-  if (!views) {
-    m.u = m.u.contiguous();
-    if (m.z.defined()) m.z = m.z.contiguous();
-  }
-  return true;
+  m.bias = c.get(bias, {m.dim}, true);
+  m.h0 = c.get(h0, {m.batch, m.dim, m.state}, true);
+  return c.ok && m.dim % m.groups == 0;
+}
+// views: u, z, B and C keep their strides
+void m1_lay(M1& m, bool views) {
+  lay({&m.delta, &m.a, &m.d, &m.bias, &m.h0});
+  if (!views) lay({&m.u, &m.z, &m.b, &m.c});
 }
 
 py::object selective_scan(py::handle u, py::handle delta, py::handle a, py::handle b,
@@ -253,9 +255,10 @@ py::object selective_scan(py::handle u, py::handle delta, py::handle a, py::hand
                           py::handle h0, bool softplus, bool reverse) {
   Call c;
   M1 m;
-  if (!m1_args(c, m, false, u, delta, a, b, cc, d, z, bias, h0)) return py::none();
+  if (!m1_args(c, m, u, delta, a, b, cc, d, z, bias, h0)) return py::none();
   RECORD_FUNCTION("arm_scan::selective_scan", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  m1_lay(m, false);
   Tensor out = empty(c, {m.batch, m.dim, m.length}), last = empty(c, {m.batch, m.dim, m.state});
   const ArmScanDims dims = m.dims();
   if (!launch(c.device, [&](void* st) {
@@ -267,20 +270,29 @@ py::object selective_scan(py::handle u, py::handle delta, py::handle a, py::hand
   return py::make_tuple(wrap(out), wrap(last));
 }
 
-// Views that arm_scan_selective_scan_views_f32 may read in place: offsets of a batch below
-// 4 GiB, and no broadcast (the custom op materialises those).
+// Views that arm_scan_selective_scan_views_f32 reads in place, by the rule it states (the
+// library refuses the rest with code 2, after the outputs are allocated), without broadcasts
+// (the custom op materialises those).
 bool views_ok(const M1& m) {
   auto fits = [&](at::IntArrayRef s) {
-    return s[0] >= 0 && s[1] >= 0 && s[2] >= 0 &&
-           4 * ((m.dim - 1) * s[1] + (m.length - 1) * s[2] + 1) < (int64_t(1) << 32);
+    return 4 * ((m.dim - 1) * s[1] + (m.length - 1) * s[2] + 1) < (int64_t(1) << 32) &&
+           60 * s[2] < (int64_t(1) << 31);
   };
   auto view_ok = [&](const Tensor& t) {
     for (int i = 0; i < 3; ++i)
       if (t.stride(i) == 0 && t.size(i) > 1) return false;
     return fits(t.strides());
   };
+  // 16-byte rows; what is not contiguous is delta's copy, or u by its strides
+  auto lies16 = [](const Tensor& t) { return !t.is_contiguous() || aligned(t); };
+  const bool whole = m.length % 4 == 0 && lies16(m.delta) && lies16(m.u);
+  // other rows: z in 16-byte runs of channels (as out is), and more than 8 states
+  const bool staged = !m.z.defined() ||
+                      (m.z.stride(1) == 1 && m.z.stride(2) % 4 == 0 && m.z.stride(0) % 4 == 0 &&
+                       aligned(m.z) && m.state > 8);
   const std::array<int64_t, 3> out{m.length * m.dim, 1, m.dim};
-  return m.dim % 16 == 0 && (m.dim / m.groups) % 16 == 0 && fits(out) && view_ok(m.u) &&
+  return m.dim % 16 == 0 && (m.dim / m.groups) % 16 == 0 && (whole || staged) &&
+         m.batch * m.groups <= 65535 && fits(out) && view_ok(m.u) &&
          (!m.z.defined() || view_ok(m.z));
 }
 
@@ -297,10 +309,11 @@ py::object selective_scan_time_major(py::handle u, py::handle delta, py::handle 
                                      bool reverse) {
   Call c;
   M1 m;
-  if (!m1_args(c, m, true, u, delta, a, b, cc, d, z, bias, h0) || !views_ok(m))
+  if (!m1_args(c, m, u, delta, a, b, cc, d, z, bias, h0) || !views_ok(m))
     return py::none();
   RECORD_FUNCTION("arm_scan::selective_scan_time_major", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  m1_lay(m, true);
   Tensor out = empty(c, {m.batch, m.length, m.dim}).transpose(1, 2);
   Tensor last = empty(c, {m.batch, m.dim, m.state});
   const ArmScanDims dims = m.dims();
@@ -323,9 +336,10 @@ py::object bidirectional(py::handle u, py::handle delta, py::handle a, py::handl
                          bool softplus) {
   Call c;
   M1 m;
-  if (!m1_args(c, m, false, u, delta, a, b, cc, d, z, bias, py::none())) return py::none();
+  if (!m1_args(c, m, u, delta, a, b, cc, d, z, bias, py::none())) return py::none();
   RECORD_FUNCTION("arm_scan::selective_scan_bidirectional", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  m1_lay(m, false);
   Tensor fwd = empty(c, {m.batch, m.dim, m.length}), bwd = empty(c, {m.batch, m.dim, m.length});
   const ArmScanDims dims = m.dims();
   if (!launch(c.device, [&](void* st) {
@@ -352,12 +366,13 @@ py::object state_update(py::handle state, py::handle x, py::handle dt, py::handl
   if (!c.ok || s.dim() != 3 || !s.is_contiguous()) return py::none();
   const int64_t batch = s.size(0), dim = s.size(1), n = s.size(2);
   const Tensor tx = c.get(x, {batch, dim}), tdt = c.get(dt, {batch, dim}),
-               ta = c.rows(a, {dim, n}), tb = c.get(b, {batch, n}), tc = c.get(cc, {batch, n}),
-               td = c.rows(d, {dim}, true), tz = c.get(z, {batch, dim}, true),
-               tbias = c.rows(bias, {dim}, true);
+               tb = c.get(b, {batch, n}), tc = c.get(cc, {batch, n}),
+               tz = c.get(z, {batch, dim}, true);
+  Tensor ta = c.get(a, {dim, n}), td = c.get(d, {dim}, true), tbias = c.get(bias, {dim}, true);
   if (!c.ok) return py::none();
   RECORD_FUNCTION("arm_scan::selective_state_update", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  lay({&ta, &td, &tbias});
   Tensor out = empty(c, {batch, dim});
   const auto xs = strides2(tx), dts = strides2(tdt), bs = strides2(tb), cs = strides2(tc);
   const auto zs = tz.defined() ? strides2(tz) : xs;
@@ -375,13 +390,15 @@ py::object state_update(py::handle state, py::handle x, py::handle dt, py::handl
 py::object causal_conv1d(py::handle x, py::handle weight, py::handle bias, bool silu,
                          bool time_major) {
   Call c;
-  const Tensor tx = c.get(x), tw0 = c.get(weight);
-  if (!c.ok || tx.dim() != 3 || tw0.dim() != 2 || tw0.size(0) != tx.size(1)) return py::none();
+  const Tensor tx = c.get(x);
+  Tensor tw = c.get(weight);
+  if (!c.ok || tx.dim() != 3 || tw.dim() != 2 || tw.size(0) != tx.size(1)) return py::none();
   const int64_t batch = tx.size(0), dim = tx.size(1), length = tx.size(2);
-  const Tensor tw = tw0.contiguous(), tb = c.rows(bias, {dim}, true);
+  Tensor tb = c.get(bias, {dim}, true);
   if (!c.ok) return py::none();
   RECORD_FUNCTION("arm_scan::causal_conv1d", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  lay({&tw, &tb});
   Tensor out = time_major ? empty(c, {batch, length, dim}).transpose(1, 2)
                           : empty(c, {batch, dim, length});
   const int64_t xs[3] = {tx.stride(0), tx.stride(1), tx.stride(2)};
@@ -396,14 +413,15 @@ py::object causal_conv1d(py::handle x, py::handle weight, py::handle bias, bool 
 py::object causal_conv1d_update(py::handle x, py::handle state, py::handle weight,
                                 py::handle bias, bool silu) {
   Call c;
-  const Tensor tx = c.get(x), tw0 = c.get(weight);
-  if (!c.ok || tx.dim() != 2 || tw0.dim() != 2 || tw0.size(0) != tx.size(1)) return py::none();
-  const int64_t batch = tx.size(0), dim = tx.size(1), width = tw0.size(1);
-  Tensor s = c.get(state, {batch, dim, width});
-  const Tensor tw = tw0.contiguous(), tb = c.rows(bias, {dim}, true);
+  const Tensor tx = c.get(x);
+  Tensor tw = c.get(weight);
+  if (!c.ok || tx.dim() != 2 || tw.dim() != 2 || tw.size(0) != tx.size(1)) return py::none();
+  const int64_t batch = tx.size(0), dim = tx.size(1), width = tw.size(1);
+  Tensor s = c.get(state, {batch, dim, width}), tb = c.get(bias, {dim}, true);
   if (!c.ok || !s.is_contiguous()) return py::none();
   RECORD_FUNCTION("arm_scan::causal_conv1d_update", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  lay({&tw, &tb});
   Tensor out = empty(c, {batch, dim});
   const int64_t xs[2] = {tx.stride(0), tx.stride(1)};
   if (!launch(c.device, [&](void* st) {
@@ -424,14 +442,13 @@ py::object ss2d(py::handle u, py::handle delta, py::handle a, py::handle b4, py:
   if (!c.ok || tu.dim() != 4 || ta.dim() != 2 || ta.size(0) != tu.size(1)) return py::none();
   const int64_t b = tu.size(0), dim = tu.size(1), h = tu.size(2), w = tu.size(3),
                 n = ta.size(1);
-  tu = tu.contiguous();
-  ta = ta.contiguous();
-  const Tensor tdt = c.rows(delta, {b, dim, h, w}), tb = c.rows(b4, {4, b, n, h, w}),
-               tc = c.rows(c4, {4, b, n, h, w}), td = c.rows(d, {dim}, true),
-               tz = c.rows(z, {b, dim, h, w}, true), tbias = c.rows(bias, {dim}, true);
+  Tensor tdt = c.get(delta, {b, dim, h, w}), tb = c.get(b4, {4, b, n, h, w}),
+         tc = c.get(c4, {4, b, n, h, w}), td = c.get(d, {dim}, true),
+         tz = c.get(z, {b, dim, h, w}, true), tbias = c.get(bias, {dim}, true);
   if (!c.ok) return py::none();
   RECORD_FUNCTION("arm_scan::ss2d_scan", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  lay({&tu, &ta, &tdt, &tb, &tc, &td, &tz, &tbias});
   Tensor out = merge == 0 ? empty(c, {4, b, dim, h, w}) : empty(c, {b, dim, h, w}), last;
   if (want_last) last = empty(c, {4, b, dim, n});
   const ArmSS2DDims dims{(size_t)b, (size_t)dim, (size_t)h, (size_t)w, (size_t)n};
@@ -454,7 +471,7 @@ struct M3 {
   }
 };
 
-// Shapes as mamba3.py's _check_shapes; v, z and the angles keep their strides.
+// Shapes as mamba3.py's _check_shapes; m3_lay makes all but v, z and the angles contiguous.
 bool m3_args(Call& c, M3& m, const py::handle& q, const py::handle& k, const py::handle& v,
              const py::handle& adt, const py::handle& dt, const py::handle& trap,
              const py::handle& qb, const py::handle& kb, const py::handle& cos,
@@ -478,32 +495,34 @@ bool m3_args(Call& c, M3& m, const py::handle& q, const py::handle& k, const py:
   m.groups = m.q.size(full - 2);
   m.dqk = m.q.size(full - 1);
   if (m.q.size(0) != m.b || m.q.size(1) != m.length || m.dqk % 2 || m.h % m.groups) return false;
-  m.q = m.q.contiguous();
-  m.k = m.k.contiguous();
-  m.adt = c.rows(adt, {m.b, m.h, m.length});
-  m.dt = c.rows(dt, {m.b, m.h, m.length});
-  m.trap = c.rows(trap, {m.b, m.h, m.length});
+  m.adt = c.get(adt, {m.b, m.h, m.length});
+  m.dt = c.get(dt, {m.b, m.h, m.length});
+  m.trap = c.get(trap, {m.b, m.h, m.length});
   if (mimo) {
-    m.qb = c.rows(qb, {m.h, m.rank, m.dqk});
-    m.kb = c.rows(kb, {m.h, m.rank, m.dqk});
-    m.psi = c.rows(psi, {m.h, m.rank, m.dv});
-    m.zeta = c.rows(zeta, {m.h, m.rank, m.dv});
-    m.phi = c.rows(phi, {m.h, m.rank, m.dv});
+    m.qb = c.get(qb, {m.h, m.rank, m.dqk});
+    m.kb = c.get(kb, {m.h, m.rank, m.dqk});
+    m.psi = c.get(psi, {m.h, m.rank, m.dv});
+    m.zeta = c.get(zeta, {m.h, m.rank, m.dv});
+    m.phi = c.get(phi, {m.h, m.rank, m.dv});
   } else {
-    m.qb = c.rows(qb, {m.h, m.dqk});
-    m.kb = c.rows(kb, {m.h, m.dqk});
+    m.qb = c.get(qb, {m.h, m.dqk});
+    m.kb = c.get(kb, {m.h, m.dqk});
   }
-  m.d = c.rows(d, {m.h}, true);
+  m.d = c.get(d, {m.h}, true);
   m.z = c.get(z, {m.b, m.length, m.h, m.dv}, true);
   if (!c.ok) return false;
   if (!cos.is_none() || !sin.is_none()) {  // then the angles are not read
-    m.cos = c.rows(cos, {m.b, m.length, m.h, m.dqk / 2});
-    m.sin = c.rows(sin, {m.b, m.length, m.h, m.dqk / 2});
+    m.cos = c.get(cos, {m.b, m.length, m.h, m.dqk / 2});
+    m.sin = c.get(sin, {m.b, m.length, m.h, m.dqk / 2});
     return c.ok && ang.is_none();
   }
   m.ang = c.get(ang);
   return c.ok && m.ang.dim() == 4 && m.ang.size(0) == m.b && m.ang.size(1) == m.length &&
          m.ang.size(2) == m.h && m.ang.size(3) >= 1 && m.ang.size(3) <= m.dqk / 2;
+}
+void m3_lay(M3& m) {
+  lay({&m.q, &m.k, &m.adt, &m.dt, &m.trap, &m.qb, &m.kb, &m.psi, &m.zeta, &m.phi, &m.d, &m.cos,
+       &m.sin});
 }
 
 // cos and sin from the raw angles (arm_scan_mamba3_angles_f32)
@@ -543,6 +562,7 @@ py::object mamba3(py::handle q, py::handle k, py::handle v, py::handle adt, py::
     return py::none();
   RECORD_FUNCTION("arm_scan::mamba3_scan", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  m3_lay(m);
   Tensor out = empty(c, {m.b, m.length, m.h, m.dv}), state, bx;
   const ArmMamba3Dims dims = m.dims();
   auto result = [&] {
@@ -566,8 +586,7 @@ py::object mamba3(py::handle q, py::handle k, py::handle v, py::handle adt, py::
       return py::none();
     return result();
   }
-  m.v = m.v.contiguous();
-  if (m.z.defined()) m.z = m.z.contiguous();
+  lay({&m.v, &m.z});
   if (carry) {
     state = empty(c, {m.b, m.h, m.dv, m.dqk});
     if (!mimo) bx = empty(c, {m.b, m.h, m.dqk});
@@ -609,8 +628,8 @@ py::object noncausal(py::handle q, py::handle k, py::handle v, py::handle adt, p
     return py::none();
   RECORD_FUNCTION("arm_scan::mamba3_noncausal", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
-  m.v = m.v.contiguous();
-  if (m.z.defined()) m.z = m.z.contiguous();
+  m3_lay(m);
+  lay({&m.v, &m.z});
   Tensor out = empty(c, {m.b, m.length, m.h, m.dv});
   const ArmMamba3Dims dims = m.dims();
   if (!m3_rotations(c, m) || !launch(c.device, [&](void* st) {
@@ -633,16 +652,17 @@ py::object grid_mamba3(py::handle q, py::handle k, py::handle v, py::handle adt,
     return py::none();
   const int64_t b = q0.size(0), H = q0.size(1), W = q0.size(2), g = q0.size(3),
                 dqk = q0.size(4), h = v0.size(3), dv = v0.size(4), r = a0.size(4);
-  if (dqk % 2 || h % g || r > dqk / 2) return py::none();
-  const Tensor tq = c.rows(q, {b, H, W, g, dqk}), tk = c.rows(k, {b, H, W, g, dqk}),
-               tv = c.rows(v, {b, H, W, h, dv}), tadt = c.rows(adt, {b, h, H, W}),
-               tdt = c.rows(dt, {b, h, H, W}), ttrap = c.rows(trap, {b, h, H, W}),
-               tqb = c.rows(qb, {h, dqk}), tkb = c.rows(kb, {h, dqk}),
-               ta = c.rows(ang, {b, H, W, h, r}), td = c.rows(d, {h}, true),
-               tz = c.rows(z, {b, H, W, h, dv}, true);
+  if (dqk % 2 || h % g || r > dqk / 2 || H > 32768 || W > 32768) return py::none();
+  Tensor tq = c.get(q, {b, H, W, g, dqk}), tk = c.get(k, {b, H, W, g, dqk}),
+         tv = c.get(v, {b, H, W, h, dv}), tadt = c.get(adt, {b, h, H, W}),
+         tdt = c.get(dt, {b, h, H, W}), ttrap = c.get(trap, {b, h, H, W}),
+         tqb = c.get(qb, {h, dqk}), tkb = c.get(kb, {h, dqk}),
+         ta = c.get(ang, {b, H, W, h, r}), td = c.get(d, {h}, true),
+         tz = c.get(z, {b, H, W, h, dv}, true);
   if (!c.ok) return py::none();
   RECORD_FUNCTION("arm_scan::mamba3_grid", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  lay({&tq, &tk, &tv, &tadt, &tdt, &ttrap, &tqb, &tkb, &ta, &td, &tz});
   Tensor out = empty(c, {b, H, W, h, dv});
   const ArmMamba3Dims dims{(size_t)b, (size_t)h,       (size_t)dv, (size_t)dqk,
                            (size_t)(H * W), (size_t)1, (size_t)g};
@@ -669,18 +689,19 @@ py::object mixer_scan(py::handle proj, py::handle dt_bias, py::handle b_norm,
   const int64_t inner = heads * headdim;
   const int64_t col_ang = 2 * inner + 2 * rank * groups * d_state + 3 * heads;
   const bool mimo = !psi.is_none();
-  const Tensor tdt = c.rows(dt_bias, {heads}), tbn = c.rows(b_norm, {d_state}),
-               tcn = c.rows(c_norm, {d_state}), tbb = c.rows(b_bias, {heads, rank, d_state}),
-               tcb = c.rows(c_bias, {heads, rank, d_state}), td = c.rows(d, {heads});
+  Tensor tdt = c.get(dt_bias, {heads}), tbn = c.get(b_norm, {d_state}),
+         tcn = c.get(c_norm, {d_state}), tbb = c.get(b_bias, {heads, rank, d_state}),
+         tcb = c.get(c_bias, {heads, rank, d_state}), td = c.get(d, {heads});
   Tensor tpsi, tzeta, tphi;
   if (mimo) {
-    tpsi = c.rows(psi, {heads, rank, headdim});
-    tzeta = c.rows(zeta, {heads, rank, headdim});
-    tphi = c.rows(phi, {heads, rank, headdim});
+    tpsi = c.get(psi, {heads, rank, headdim});
+    tzeta = c.get(zeta, {heads, rank, headdim});
+    tphi = c.get(phi, {heads, rank, headdim});
   }
   if (!c.ok || row != col_ang + n_angles) return py::none();
   RECORD_FUNCTION("arm_scan::mamba3_mixer_scan", std::vector<c10::IValue>());
   c10::DeviceGuard on_device(c.device);
+  lay({&tdt, &tbn, &tcn, &tbb, &tcb, &td, &tpsi, &tzeta, &tphi});
   Tensor q = empty(c, {b, length, rank, groups, d_state}),
          k = empty(c, {b, length, rank, groups, d_state}), adt = empty(c, {b, heads, length}),
          dt = empty(c, {b, heads, length}), trap = empty(c, {b, heads, length}),

@@ -227,6 +227,95 @@ def test_scratch_during_capture():
         assert torch.equal(run(), want)
 
 
+def _allocations():
+    import torch
+
+    return torch.cuda.memory_stats()["allocation.all.allocated"]
+
+
+def test_refusals_allocate_nothing():
+    """What is left to the custom op has been copied and allocated by nobody yet."""
+    import torch
+
+    from armhackathon_amd import op
+
+    f, no = op.front(), (None,) * 4
+    b, d, n, L = 2, 32, 16, 77
+    u, A, B = _rand(b, d, L), -torch.rand(n, d, device="cuda").t(), _rand(b, L, n).transpose(1, 2)
+    tm = _rand(b, L, d).transpose(1, 2)  # as delta: a copy where it is taken
+    few, B8 = -torch.rand(d, 8, device="cuda"), _rand(b, 8, L)
+    grid, B4 = _rand(b, d, 7, 7), _rand(4, b, n, 7, 7)
+    q, v, g = _rand(b, 64, L).transpose(1, 2), _rand(b, L, 4, 32), _rand(b, 4, L)
+    bias, cos = _rand(4, 64), _rand(b, L, 4, 32)
+    wants_grad, state = torch.nn.Parameter(bias.clone()), torch.zeros(b, d, n, device="cuda")
+    refused = {
+        "dim 24": lambda: f.selective_scan_time_major(tm[:, :24], tm[:, :24], A[:24], B, B, *no,
+                                                      True, False),
+        "8 states, odd rows": lambda: f.selective_scan_time_major(
+            tm, tm, few, B8, B8, None, tm, None, None, True, False),
+        "z not by channels": lambda: f.selective_scan_time_major(tm, tm, A, B, B, None, u, None,
+                                                                 None, True, False),
+        "scan, h0 of another shape": lambda: f.selective_scan(tm, tm, A, B, B, None, tm, None,
+                                                              u, True, False),
+        "ss2d, z of another shape": lambda: f.ss2d(grid.transpose(2, 3), grid, A, B4, B4, None,
+                                                   u, None, True, 1, False),
+        "mamba3, a gradient": lambda: f.mamba3(q, q, v, g, g, g, bias, wants_grad, cos, cos, None,
+                                               *no, None, False, False, False),
+        "step, z of another shape": lambda: f.state_update(
+            state, u[..., 0], u[..., 1], A, B[..., 0], B[..., 0], None, u, None, True),
+    }
+    for name, call in refused.items():
+        case(f"refused: {name}")
+        before = _allocations()
+        assert call() is None
+        assert _allocations() == before, name
+
+
+def test_views_rule_is_the_library_s():
+    """The front-end takes a time-major call where the library's views entry does."""
+    import ctypes
+    import itertools
+
+    import torch
+
+    from armhackathon_amd import _ffi, op
+
+    f, lib, b, d = op.front(), _ffi.load(), 2, 32
+
+    def strides(t, k):
+        return (ctypes.c_longlong * k)(*t.stride())
+
+    def layouts(L):
+        wide = _rand(b, L, 2 * d + 4, seed=L)
+        flat = _rand(b * d * L + 1, seed=L + 1)
+        return {"rows": _rand(b, d, L), "rows, off 16 bytes": flat[1:].view(b, d, L),
+                "columns": wide[..., :d].transpose(1, 2),
+                "columns, off 16 bytes": wide[..., 1:1 + d].transpose(1, 2),
+                "columns, odd steps": _rand(b, L, d + 1)[..., :d].transpose(1, 2)}
+
+    taken = set()
+    for L, n in itertools.product((1, 64, 77), (8, 16)):
+        A, B = -torch.rand(d, n, device="cuda"), _rand(b, 1, n, L)
+        x = layouts(L)
+        for un, zn, dn in itertools.product(x, [None, *x], ("rows", "rows, off 16 bytes")):
+            case(f"views L {L} states {n}: u {un}, z {zn}, delta {dn}")
+            u, delta, z = x[un], x[dn], None if zn is None else x[zn]
+            got = f.selective_scan_time_major(u, delta, A, B, B, None, z, None, None, True, False)
+            out = torch.empty(b, L, d, device="cuda").transpose(1, 2)
+            rc = lib.arm_scan_selective_scan_views_f32(
+                ctypes.byref(_ffi.ArmScanDims(b, d, L, n, 1)), u.data_ptr(),
+                None if u.is_contiguous() else strides(u, 3), delta.data_ptr(), A.data_ptr(),
+                B.data_ptr(), strides(B, 4), B.data_ptr(), strides(B, 4), None,
+                None if z is None else z.data_ptr(), None if z is None else strides(z, 3), None,
+                1, 0, out.data_ptr(), strides(out, 3), None, None,
+                torch.cuda.current_stream().cuda_stream)
+            assert rc in (0, 2) and (got is None) == (rc == 2)
+            if rc == 0:
+                assert torch.equal(got[0], out)
+            taken.add(rc)
+    assert taken == {0, 2}
+
+
 def _node_types(graph):
     import ctypes
 
