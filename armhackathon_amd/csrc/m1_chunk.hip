@@ -1242,22 +1242,30 @@ m1_tile_jobs_kernel(M1Kern p, M1Jobs jobs) {
   else tile_rows<I, false, 0, false, ALN, TAIL>(p, blk);
 }
 
+// Floats of LDS of a block: two tiles, the stage of z and out where they pass through it, and
+// the per-state values of 16 rows, three of the fold pass and two of the scan.
+template <int I>
+constexpr size_t fold_lds_floats(size_t N) {
+  return 2 * (size_t)Tile<I>::FLOATS + 3 * 16 * N;
+}
+template <int I>
+constexpr size_t tile_lds_floats(size_t N, bool staged) {
+  return 2 * (size_t)Tile<I>::FLOATS + (staged ? kZStageFloats : 0) + (2 * 16 + 1) * N + kZerosPad;
+}
+
 template <int I, bool REV, int SIO, bool ALN, bool DWBC>
 hipError_t launch_tile(const M1Kern& k, hipStream_t st) {
-  constexpr int RPB = kWavesPerBlock * 4;
-  const long long blocks = (long long)k.rows / RPB;
+  const long long blocks = (long long)k.rows / 16;
   const int segs = k.segs > 1 ? k.segs : 1;
   if (segs > 1) {  // pass 1: the maps of segments 0 .. segs-2
-    const size_t lds1 = sizeof(float) * (2 * (size_t)Tile<I>::FLOATS + 3 * (size_t)RPB * k.N);
+    const size_t lds1 = sizeof(float) * fold_lds_floats<I>(k.N);
     hipLaunchKernelGGL((m1_seg_fold_kernel<I, REV, ALN, DWBC>),
                        dim3((unsigned)(blocks * (segs - 1))),
                        dim3(64 * kWavesPerBlock), lds1, st, k);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  const size_t lds =
-      sizeof(float) * (2 * (size_t)Tile<I>::FLOATS + (SIO >= 2 || !ALN ? kZStageFloats : 0) +
-                       (2 * (size_t)RPB + 1) * k.N + kZerosPad);
+  const size_t lds = sizeof(float) * tile_lds_floats<I>(k.N, SIO >= 2 || !ALN);
   const dim3 grid((unsigned)(segs > 1 ? blocks * segs : blocks)), wg(64 * kWavesPerBlock);
   const bool tail = k.L % Tile<I>::CH != 0;
   auto go = [&](auto seg_tag, auto tail_tag) {
@@ -1323,9 +1331,7 @@ hipError_t m1_scan_jobs(const M1Problem& pr, const M1JobSpec* spec, int n, hipSt
     jobs.job[i] = M1Job{j.u, j.delta, j.z, j.B, j.C, j.out, j.last, j.rev};
   }
   const long long blocks = 8LL * n * ((jobs.blocks_per_job + 7) / 8);
-  const size_t lds = sizeof(float) * (2 * (size_t)Tile<M1_TILE_I>::FLOATS +
-                                      (aln ? 0 : kZStageFloats) + (2 * (size_t)16 + 1) * k.N +
-                                      kZerosPad);
+  const size_t lds = sizeof(float) * tile_lds_floats<M1_TILE_I>(k.N, !aln);
   const bool tail = k.L % Tile<M1_TILE_I>::CH != 0;
   const dim3 grid((unsigned)blocks), wg(64 * kWavesPerBlock);
   if (aln && tail)
@@ -1381,18 +1387,26 @@ hipError_t m1_noalloc_scratch(float** out, size_t* bytes) {
 
 namespace {
 // Modelled time of a scan of `blocks` row blocks cut into `segs` segments, in microseconds:
-// rounds of 768 resident blocks (three a CU), each as long as its chunks take with one, two
-// or three blocks on a CU (9.1, 11.7 and 15.6 us a chunk at N 16, from B1 to B8 D1536 L2048)
-// and 3 us of start, the last segment's further chunks (the row's tail) on its own blocks;
-// before them the fold of all segments but the last at 0.75 of that, and 4 us for the second
-// launch. Within 10% of what was measured below, but for several rounds (15%).
-double plan_cost(long long blocks, long long segs, long long nfull, bool tail, int N) {
+// rounds of resident blocks, `per_cu` a CU, each as long as its chunks take with one, two or
+// three blocks on a CU (9.1, 11.7 and 15.6 us a chunk at N 16) and 3 us of start, a further
+// round's by N (the states its blocks begin and end with), the last segment's further chunks
+// (the row's tail) on its own blocks; before them the fold of all segments but the last at
+// 0.75 of that, `fold_per_cu` blocks a CU, and 4 us for the second launch. Only the order of
+// the plans counts: over 724 sizes (contiguous and time-major, N 12 to 256, 96 to 480 blocks,
+// L 1024 to 8192, one to eight segments each) the plan taken is 0.9% from the fastest on
+// average and 18% at most, and 2.7 to 4% behind ceil(768 / blocks) segments at three sizes.
+// With three blocks a CU whatever their LDS, and 3 us for any round, it was 3.7% and 76%: N 128
+// of 256 blocks at L 4096 took eight segments, 940 us for 798 with three, time-major N 48 of
+// 224 blocks at L 8192 three, 800 for 704 with four.
+double plan_cost(long long blocks, long long segs, long long nfull, bool tail, int N, int per_cu,
+                 int fold_per_cu) {
   static const double chunk_us[4] = {0.0, 9.1, 11.7, 15.6};
-  auto pass = [&](long long nblk, double chunks, double weight) {
+  const double by_n = N / 16.0;
+  auto pass = [&](long long nblk, double chunks, double weight, int most) {
     double t = 0.0;
-    for (long long left = nblk; left > 0; left -= 768) {
-      const long long per_cu = left >= 768 ? 3 : (left + 255) / 256;
-      t += weight * chunks * chunk_us[per_cu] * N / 16.0 + 3.0;
+    for (long long left = nblk; left > 0; left -= 256 * most) {
+      const long long on = left >= 256 * most ? most : (left + 255) / 256;
+      t += weight * chunks * chunk_us[on] * by_n + 3.0 * (t > 0.0 && by_n > 1.0 ? by_n : 1.0);
     }
     return t;
   };
@@ -1400,21 +1414,28 @@ double plan_cost(long long blocks, long long segs, long long nfull, bool tail, i
   segs = (nfull + len - 1) / len;  // as many as segments of that length need
   const long long last = nfull - (segs - 1) * len + (tail ? 1 : 0);
   const long long alone = (blocks + 255) / 256;  // blocks a CU once only the last one runs
-  const double t = pass(blocks * segs, (double)len, 1.0) +
-                   (last > len ? (last - len) * chunk_us[alone > 3 ? 3 : alone] * N / 16.0 : 0.0);
-  return segs == 1 ? t : t + pass(blocks * (segs - 1), (double)len, 0.75) + 4.0;
+  const double t = pass(blocks * segs, (double)len, 1.0, per_cu) +
+                   (last > len ? (last - len) * chunk_us[alone > 3 ? 3 : alone] * by_n : 0.0);
+  return segs == 1 ? t : t + pass(blocks * (segs - 1), (double)len, 0.75, fold_per_cu) + 4.0;
+}
+
+// Blocks of `floats` of LDS that a CU holds, at most the three of the launch bounds.
+int blocks_per_cu(size_t floats) {
+  const size_t n = 160 * 1024 / (sizeof(float) * floats);
+  return n > 3 ? 3 : n < 1 ? 1 : (int)n;
 }
 
 // Rows cut into segments when there are too few to fill the chip: a 16-row block per
-// CU slot, 768 slots (three per CU) resident at once, as many segments as the model above
+// CU slot, at most 768 slots (three per CU) resident at once, as many segments as the model above
 // finds fastest (whole rows among them). B4 L1531 and L4096 with the convolution 127 -> 112
 // and 287 -> 258 us, B3 L1000 82 -> 70 (whole rows: two blocks a CU already, and no fold
-// pass), B3 L8192 alone 362 -> 311 (eight segments: three even rounds); B1 and B2 L2048 keep
+// pass), B3 L8192 alone 355 -> 292 (eight segments: three even rounds); B1 and B2 L2048 keep
 // eight and four. Sets k.segs / k.seg_chunks and
 // allocates the segment maps on the stream, or, with caller scratch, takes them from
 // it, cutting the plan to fewer segments (down to whole rows, which need no maps)
 // until they fit.
-hipError_t plan_segments(M1Kern& k, float* scratch_p, size_t scratch_bytes, hipStream_t st) {
+hipError_t plan_segments(M1Kern& k, bool staged, float* scratch_p, size_t scratch_bytes,
+                         hipStream_t st) {
   static_assert(16 * M1_TILE_I == kM1ChunkSteps, "chunk size shared with the ABI's routing");
   const long long blocks = k.rows / 16;
   const long long nfull = k.L / (16 * M1_TILE_I);
@@ -1427,9 +1448,11 @@ hipError_t plan_segments(M1Kern& k, float* scratch_p, size_t scratch_bytes, hipS
   if (most > nfull) most = nfull;
   long long segs = 1;
   const bool tail = k.L % (16 * M1_TILE_I) != 0;
-  double best = plan_cost(blocks, 1, nfull, tail, k.N);
+  const int per_cu = blocks_per_cu(tile_lds_floats<M1_TILE_I>(k.N, staged));
+  const int fold_per_cu = blocks_per_cu(fold_lds_floats<M1_TILE_I>(k.N));
+  double best = plan_cost(blocks, 1, nfull, tail, k.N, per_cu, fold_per_cu);
   for (long long s = 2; s <= most; ++s) {
-    const double c = plan_cost(blocks, s, nfull, tail, k.N);
+    const double c = plan_cost(blocks, s, nfull, tail, k.N, per_cu, fold_per_cu);
     if (c < 1.03 * best) {  // near ties: the finer cut, whose blocks end together
       best = c < best ? c : best;
       segs = s;
@@ -1458,7 +1481,7 @@ hipError_t plan_segments(M1Kern& k, float* scratch_p, size_t scratch_bytes, hipS
 template <int SIO, bool ALN = true, bool DWBC = false>
 hipError_t run_tile(M1Kern& k, bool rev, float* scratch_p, size_t scratch_bytes,
                     hipStream_t st) {
-  hipError_t e = plan_segments(k, scratch_p, scratch_bytes, st);
+  hipError_t e = plan_segments(k, SIO >= 2 || !ALN, scratch_p, scratch_bytes, st);
   if (e != hipSuccess) return e;
   e = rev ? launch_tile<M1_TILE_I, true, SIO, ALN, DWBC>(k, st)
           : launch_tile<M1_TILE_I, false, SIO, ALN, DWBC>(k, st);
