@@ -227,6 +227,26 @@ def test_scratch_during_capture():
         assert torch.equal(run(), want)
 
 
+@pytest.mark.parametrize("native", [True, False], ids=["front-end", "custom op"])
+def test_autocast_changes_nothing(native, monkeypatch):
+    """The ops have no autocast rule: a float32 call is the same under it, on either route."""
+    import torch
+
+    from armhackathon_amd import op
+
+    if not native:
+        monkeypatch.setattr(op, "front", lambda: None)
+    calls = _calls()
+    for name in ("scan_views", "bidir", "m3_cos"):
+        case(f"autocast, {'front-end' if native else 'custom op'}: {name}")
+        want = calls[name]()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            got = calls[name]()
+        flat = lambda r: r if isinstance(r, tuple) else (r,)  # noqa: E731
+        for g, w in zip(flat(got), flat(want)):
+            assert g.dtype == torch.float32 and torch.equal(g, w)
+
+
 def _allocations():
     import torch
 

@@ -2,10 +2,13 @@
 of 1 to 16 lanes a row, blocks whose last rows are missing, B and C by pieces or by strides,
 a window of another width or alignment (the one-thread kernels).
 
-Gate 2e-6 of the sum of the absolute terms of the largest output, which is what bounds the
-rounding of a 32-bit sum whose terms cancel (a single row's y may be small beside them): up
-to 144 products and roundings of 2^-24 each (8.6e-6 at worst, their square root, 7e-7,
-typical) of states that one 32-bit exponential and two roundings make.
+Every element is held to the bound of its own roundings, in units e = 2^-24 of its terms'
+absolute values (an output may be small beside terms that cancel):
+- dt = softplus(s): s rounded (|s| e), exp by exp2 of a rounded argument (2 |s| e, and 2 e for
+  exp2's own ulp), log1p 6 e: (3 |s| + 8) e;
+- exp(dt A): the relative error of dt and three roundings of the argument, times |dt A|, and
+  2 e; the state two more: (3 |s| + 12) e of e^{dt A} |h| (1 + |dt A|) + |dt x B|;
+- y: the states' errors and up to 45 e of sums (144 states on four lanes), silu (2 |z| + 6) e.
 """
 
 import pytest
@@ -36,13 +39,18 @@ def test_state_update(n, rows, columns):
     dt64 = torch.nn.functional.softplus(f(dt) + f(bias))
     want_h = torch.exp(dt64[..., None] * f(A)) * f(h) + (dt64 * f(x))[..., None] * f(B)[:, None]
     want = ((want_h * f(C)[:, None]).sum(-1) + f(D) * f(x)) * torch.nn.functional.silu(f(z))
-    terms_h = (torch.exp(dt64[..., None] * f(A)) * f(h)).abs() \
-        + ((dt64 * f(x))[..., None] * f(B)[:, None]).abs()
-    terms = ((terms_h * f(C)[:, None].abs()).sum(-1) + (f(D) * f(x)).abs()) \
-        * torch.nn.functional.silu(f(z)).abs()
+    decayed = (torch.exp(dt64[..., None] * f(A)) * f(h)).abs()
+    inflow = ((dt64 * f(x))[..., None] * f(B)[:, None]).abs()
+    err_h = (3 * (f(dt) + f(bias)).abs() + 12)[..., None] \
+        * (decayed * (1 + (dt64[..., None] * f(A)).abs()) + inflow)
+    silu = torch.nn.functional.silu(f(z)).abs()
+    terms = (decayed + inflow) * f(C)[:, None].abs()
+    skip = (f(D) * f(x)).abs()
+    err_y = silu * ((err_h * f(C)[:, None].abs()).sum(-1) + 45 * (terms.sum(-1) + skip)
+                    + (2 * f(z).abs() + 6) * (terms.sum(-1) + skip))
     y = arm.selective_state_update(h, x, dt, A, B, C, D=D, z=z, dt_bias=bias, dt_softplus=True)
-    for got, ref, scale in ((y, want, terms), (h, want_h, terms_h)):
-        assert ((got.double() - ref).abs().max() / scale.max()).item() < 2e-6
+    for got, ref, err in ((y, want, err_y), (h, want_h, err_h)):
+        assert ((got.double() - ref).abs() / err).max().item() < 2.0 ** -24
 
 
 @pytest.mark.parametrize("width,offset", [(4, 0), (4, 1), (3, 0), (8, 0)])
@@ -62,5 +70,8 @@ def test_conv_step(width, offset, rows):
     want = torch.nn.functional.silu((win.double() * w.double()).sum(-1) + bias.double())
     y = arm.causal_conv1d_update(x, s, w, bias, activation="silu")
     assert torch.equal(s, win)
+    # the sum (a rounding a tap), through silu's slope of at most 1.1, and silu itself
+    acc = (win.double() * w.double()).sum(-1) + bias.double()
     terms = (win.double() * w.double()).abs().sum(-1) + bias.double().abs()
-    assert ((y.double() - want).abs().max() / terms.max()).item() < 2e-6
+    err = 1.1 * (width + 1) * terms + (2 * acc.abs() + 6) * want.abs()
+    assert ((y.double() - want).abs() / err).max().item() < 2.0 ** -24

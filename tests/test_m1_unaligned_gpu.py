@@ -15,17 +15,12 @@ from util import case, host, rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("length", [1, 2, 3, 5, 6, 7, 17, 18, 19, 31, 253, 254, 255, 257, 259,
-                                    511, 769, 1538])
-@pytest.mark.parametrize("reverse", [False, True])
-@pytest.mark.parametrize("pair", [False, True])
-def test_row_ends(length, reverse, pair):
-    """pair: both directions in one launch (bidirectional), whose reverse one is checked too."""
+LENGTHS = [1, 2, 3, 5, 6, 7, 17, 18, 19, 31, 253, 254, 255, 257, 259, 511, 769, 1538]
+
+
+def _inputs(length):
     import torch
 
-    import armhackathon_amd as arm
-
-    case(f"unaligned rows L {length} reverse={reverse} pair={pair}")
     rng = np.random.default_rng(length)
     b, d, n = 2, 32, 16
     f = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
@@ -33,12 +28,33 @@ def test_row_ends(length, reverse, pair):
              B=f(b, n, length), C=f(b, n, length), D=f(d), z=f(b, d, length), bias=f(d))
     t = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in x.items()}
     kw = dict(D=t["D"], z=t["z"], delta_bias=t["bias"], delta_softplus=True)
-    args = [t[k] for k in ("u", "delta", "A", "B", "C")]
-    want, last = naive.m1_scan(x["u"], x["delta"], x["A"], x["B"], x["C"], D=x["D"], z=x["z"],
-                               delta_bias=x["bias"], delta_softplus=True, reverse=reverse)
-    if pair:
-        out = arm.bidirectional_scan(*args, merge="none", **kw)[int(reverse)]
-    else:
-        out, got = arm.selective_scan(*args, reverse=reverse, return_last_state=True, **kw)
-        assert rel_err(host(got), last) < 2e-6
+    return x, [t[k] for k in ("u", "delta", "A", "B", "C")], kw
+
+
+def _want(x, reverse):
+    return naive.m1_scan(x["u"], x["delta"], x["A"], x["B"], x["C"], D=x["D"], z=x["z"],
+                         delta_bias=x["bias"], delta_softplus=True, reverse=reverse)
+
+
+@pytest.mark.parametrize("length", LENGTHS)
+@pytest.mark.parametrize("reverse", [False, True])
+def test_row_ends(length, reverse):
+    import armhackathon_amd as arm
+
+    case(f"unaligned rows L {length} reverse={reverse}")
+    x, args, kw = _inputs(length)
+    want, last = _want(x, reverse)
+    out, got = arm.selective_scan(*args, reverse=reverse, return_last_state=True, **kw)
+    assert rel_err(host(got), last) < 2e-6
     assert rel_err(host(out), want) < 2e-6
+
+
+@pytest.mark.parametrize("length", LENGTHS)
+def test_row_ends_of_a_pair(length):
+    """Both directions in one launch."""
+    import armhackathon_amd as arm
+
+    case(f"unaligned rows L {length}, both directions")
+    x, args, kw = _inputs(length)
+    for out, reverse in zip(arm.bidirectional_scan(*args, merge="none", **kw), (False, True)):
+        assert rel_err(host(out), _want(x, reverse)[0]) < 2e-6

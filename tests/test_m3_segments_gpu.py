@@ -38,12 +38,15 @@ CASES = [
     # (rank or 0 for SISO, batch, length, heads, dv, dqk, groups)
     (0, 1, 368, 3, 64, 128, 1),    # 23 chunks: whole
     (0, 1, 369, 3, 64, 128, 3),    # 24, the last of one step: the shortest cut
-    (0, 1, 1033, 1, 32, 128, 1),   # one block a sequence, the most segments and pieces
+    (0, 1, 1033, 1, 32, 128, 1),   # 13 segments of five chunks, one block each
+    (0, 1, 3000, 1, 32, 128, 1),   # 47 segments, more pieces than a segment's cap, one XCD
+    (0, 1, 2304, 12, 32, 64, 1),   # 12 sequences: uneven over the XCDs, in several rounds
     (0, 2, 900, 24, 64, 128, 1),   # 96 blocks: two segments
     (0, 1, 1500, 24, 64, 64, 1),   # 48 blocks: segments rounded up to whole pieces
     (2, 1, 261, 5, 64, 128, 5),
     (4, 1, 93, 3, 64, 128, 1),     # 24 chunks of four steps
     (4, 2, 530, 8, 64, 64, 1),
+    (4, 1, 1100, 1, 32, 64, 1),    # 275 chunks: 55 segments
 ]
 
 
