@@ -216,8 +216,10 @@ hipError_t stream_alloc(void** p, size_t bytes, hipStream_t st) {
 }
 
 hipError_t stream_free(void* p, hipStream_t st) {
+  // a block of the thread's own source is its owner's to give back, after the call: all of a
+  // call's blocks live to its end (a causal grid call holds both traversals' records at once)
   for (int i = 0; i < t_scratch.n; ++i)
-    if (t_scratch.given[i] == p) return hipSuccess;  // its owner gives it back
+    if (t_scratch.given[i] == p) return hipSuccess;
   return hipFreeAsync(p, st);
 }
 

@@ -833,7 +833,7 @@ __device__ __forceinline__ void tile_rows(const M1Kern& p, long long blk, int se
 
   // A lane block of a contiguous row. Aligned rows: 16-byte pieces, where in the
   // tail chunk a piece past the row's end (L % 4 == 0: a piece lies wholly in or
-  // out) reads kZeroPiece; otherwise single floats, bounds-checked in the tail.
+  // out) reads kZeroPiece; otherwise by load_unaligned.
   auto load_c = [&](const float* r, long long sbl, bool full, float (&v)[I]) {
     if constexpr (ALN) {
       const long long mb = REV ? L - sbl - I : sbl;  // the block's lowest memory step
@@ -1306,8 +1306,8 @@ bool aligned16(const void* q) { return q == nullptr || ((uintptr_t)q & 15u) == 0
 
 }  // namespace
 
-// Rows of any length and alignment: unaligned ones (L % 4 != 0 or a base off 16 bytes)
-// take the single-float instantiation.
+// Rows of any length and alignment: unaligned ones (L % 4 != 0 or a base off 16 bytes) take
+// the instantiation that loads them by load_unaligned and fills B/C tiles by single floats.
 bool m1_jobs_supported(const M1Problem& pr) {
   return pr.dim % 16 == 0 && pr.groups == 1 && pr.h0 == nullptr;
 }

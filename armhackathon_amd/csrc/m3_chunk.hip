@@ -86,8 +86,9 @@ constexpr int kMinSplitChunks = 64;
 constexpr int kMinSplitChunksRank1 = 256;
 constexpr int kFoldStages = 8;       // deepest DMA ring of the fold pass
 // Equal segments (at most half as many blocks as CUs): from this many chunks, of at least
-// this many each, folded in pieces of at least this many, and at most this many pieces in
-// all for the last segment's blocks to combine
+// this many each. A segment is folded in pieces of at least kMinPieceChunks, in more than one
+// only while the pieces are at most kMaxPieces in all; more segments than that, up to one a CU,
+// have one piece each, which the last segment's blocks combine one after another
 constexpr int kMinEqualChunks = 24;
 constexpr int kMinSegChunks = 4;
 constexpr int kMinPieceChunks = 4;
@@ -1465,8 +1466,12 @@ hipError_t m3_scan_chunked(const M3Problem& pr, hipStream_t st) {
   // (the state update alone, in pieces, many at once), then the scan runs every segment's
   // blocks, each starting from the pieces before it.
   //
-  // Up to C / 2 blocks: floor(C / P) equal segments, so that all blocks run at once. Rank
-  // 1, H24 dv64 dqk128, one sequence of L (time of a call): L 512 50 -> 37 us, 1024 86 -> 54,
+  // Up to C / 2 blocks: floor(C / P) equal segments, one block a CU. A sequence's blocks
+  // share an XCD, so they all run at once only if the sequences spread evenly over the XCDs
+  // (a multiple of 8); otherwise the fullest XCD takes several rounds, up to eight for one
+  // sequence of 256 segments, which is still less than whole sequences: one of dv32 L 16384
+  // 708 -> 460 us, of dv16 dqk16 700 -> 647, three of dv64 L 2048 139 -> 51, twelve of L 8192
+  // 305 -> 173. Rank 1, H24 dv64 dqk128, one sequence of L (time of a call): L 512 50 -> 37 us, 1024 86 -> 54,
   // 2048 158 -> 78, 4096 187 -> 120; rank 4: L 128 47 -> 34, 512 100 -> 72; rank 4 and 8
   // heads of L 512 112 -> 41. The fold pass and a second start of the ring cost about 12
   // us, so the cuts start at 24 chunks (16: 33 against 31 us of kernels, less than the

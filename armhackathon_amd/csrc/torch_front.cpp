@@ -14,7 +14,9 @@
 // Python caller then goes through the custom op, which checks, raises and dispatches as
 // it always did. Plain means: CUDA float32 strided tensors of torch's own classes on one
 // device, no gradient to record, no forward-mode tangent, and nothing between the caller
-// and the kernels (no dispatch or function mode, functorch transform, tracer, autocast).
+// and the kernels (no dispatch or function mode, functorch transform, tracer). Autocast is not
+// looked at: the ops have no autocast rule, and float32 arguments stay float32 under it on
+// either route.
 // A shape or argument that a check would refuse is not plain either, nor is an error from
 // the C ABI: the custom op's own path reports both.
 //
