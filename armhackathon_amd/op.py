@@ -62,9 +62,9 @@ class _on(torch.cuda.device):
     graph then; the library's own pool does not serve a capture."""
 
     def __enter__(self):
+        lib = _ffi.load()  # may raise: before the device is set
         super().__enter__()
         self._held = None
-        lib = _ffi.load()
         if torch.cuda.is_current_stream_capturing() and hasattr(lib, "arm_scan_thread_scratch"):
             self._held = []
 

@@ -56,3 +56,20 @@ def test_absent_front_end_leaves_the_custom_op(why, tmp_path, monkeypatch):
     with warnings.catch_warnings():
         warnings.simplefilter("error")  # told once
         assert _front.front() is None
+
+
+def test_missing_library_leaves_the_device(monkeypatch):
+    """The loader's error comes before the call's device is made current."""
+    from armhackathon_amd import op
+
+    entered = []
+    monkeypatch.setattr(torch.cuda.device, "__enter__", lambda self: entered.append(self))
+
+    def missing():
+        raise OSError("no library")
+
+    monkeypatch.setattr(_ffi, "load", missing)
+    with pytest.raises(OSError, match="no library"):
+        with op._on(torch.device("cuda", 0)):
+            pass
+    assert not entered
