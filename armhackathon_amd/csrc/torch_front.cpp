@@ -154,7 +154,7 @@ struct Call {
 // call that goes on to the custom op, which makes them too, has paid for none here.
 void lay(std::initializer_list<Tensor*> ts) {
   for (Tensor* t : ts)
-    if (t->defined()) *t = t->contiguous();
+    if (t->defined() && !t->is_contiguous()) *t = t->contiguous();
 }
 
 const float* ptr(const Tensor& t) { return t.defined() ? t.const_data_ptr<float>() : nullptr; }
