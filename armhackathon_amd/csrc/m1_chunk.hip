@@ -185,10 +185,13 @@ __device__ __forceinline__ void load_block(const float* __restrict__ row, long l
 
 // The I steps of a lane block of a contiguous row at any float address, by 16-byte loads:
 // global loads need 4-byte alignment only, and as single floats a wave's 16 loads touched 64
-// lines each (B8 D1536 L2047 144 -> 136 us, bidirectional B16 D192 L197 26.1 -> 23.1). In the
+// lines each (B8 D1536 L2047 144 -> 136 us, bidirectional B16 D192 L197 26.1 -> 22.9). In the
 // row's tail (`full` false) a piece that crosses the row's end is read from the row's last
 // four floats and shifted, so that no load branches; steps past the end read 0. Rows of fewer
-// than four steps go by single floats.
+// than four steps go by three single floats. A tail of few steps pays for the shifts: with 64-bit
+// positions and sixteen single floats for the shortest rows, bidirectional B128 D768 N4 took 141
+// us at L 3, 148 at L 21, as single floats 130 and 134; now 128 and 141 (N 16: 290 and 289, 275
+// and 279, now 273 and 285). A branch past the lanes that lie outside the row gained nothing.
 typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
 template <int I, bool REV>
 __device__ __forceinline__ void load_unaligned(const float* __restrict__ row, long long L,
@@ -196,25 +199,29 @@ __device__ __forceinline__ void load_unaligned(const float* __restrict__ row, lo
   const long long mb = REV ? L - sb - I : sb;  // the block's lowest memory step
   if (!full && L < 4) {                        // wave-uniform
 #pragma unroll
-    for (int i = 0; i < I; ++i) v[i] = sb + i < L ? row[REV ? L - 1 - sb - i : sb + i] : 0.0f;
+    for (int i = 0; i < I; ++i)  // the first lane block's first three at most
+      v[i] = i < 3 && sb + i < L ? row[REV ? L - 1 - sb - i : sb + i] : 0.0f;
     return;
   }
+  const float* base = row + mb;
+  const int rem = full ? I : (int)(L - sb);  // the block's steps, negative past the row
 #pragma unroll
   for (int q = 0; q < I / 4; ++q) {
-    const long long m = mb + 4 * q;
-    // the four floats read: at m, moved inside the row (down forward, up reverse)
-    const long long at = full ? m : REV ? (m > 0 ? m : 0) : (m < L - 4 ? m : L - 4);
-    const float4_any x = *reinterpret_cast<const float4_any*>(row + at);
+    // the piece's four floats, moved inside the row (down forward, up reverse) by `off`; 4 and
+    // more: all of them are outside
+    const int out = REV ? I - 4 * q - rem : 4 * q + 4 - rem;
+    const int off = out > 0 ? out : 0;
+    const float4_any x =
+        *reinterpret_cast<const float4_any*>(base + (REV ? 4 * q + off : 4 * q - off));
     float w[4] = {x[0], x[1], x[2], x[3]};
     if (!full) {
-      const long long off = REV ? at - m : m - at;  // by this many; 4 and more: all outside
       const bool s1 = off == 1, s2 = off == 2, s3 = off == 3, s0 = off == 0;
-      if (REV) {  // w[e] = row[m + e] = x[e - off], 0 below the row
+      if (REV) {  // w[e] = x[e - off], 0 below the row
         w[3] = s0 ? x[3] : s1 ? x[2] : s2 ? x[1] : s3 ? x[0] : 0.0f;
         w[2] = s0 ? x[2] : s1 ? x[1] : s2 ? x[0] : 0.0f;
         w[1] = s0 ? x[1] : s1 ? x[0] : 0.0f;
         w[0] = s0 ? x[0] : 0.0f;
-      } else {  // w[e] = row[m + e] = x[e + off], 0 past the row
+      } else {  // w[e] = x[e + off], 0 past the row
         w[0] = s0 ? x[0] : s1 ? x[1] : s2 ? x[2] : s3 ? x[3] : 0.0f;
         w[1] = s0 ? x[1] : s1 ? x[2] : s2 ? x[3] : 0.0f;
         w[2] = s0 ? x[2] : s1 ? x[3] : 0.0f;
