@@ -56,8 +56,8 @@ def _stream(dev):
     return torch.cuda.current_stream(dev).cuda_stream
 
 
-class _on(torch.cuda.device):
-    """The device of a library call made through ctypes. While the current stream is being
+class _CaptureAware(torch.cuda.device):
+    """The device of a library call made through ctypes. While its current stream is being
     captured the call's scratch comes from torch's allocator, whose blocks belong to the
     graph then; the library's own pool does not serve a capture."""
 
@@ -84,6 +84,14 @@ class _on(torch.cuda.device):
             _ffi.load().arm_scan_thread_scratch(None, None)
             self._held = self._alloc = None
         return super().__exit__(*exc)
+
+
+def _on(dev):
+    """The device of a library call: torch's own context unless a capture has to be looked
+    for behind it (2 us of a call's host time)."""
+    if dev.index == torch.cuda.current_device() and not torch.cuda.is_current_stream_capturing():
+        return torch.cuda.device(dev)
+    return _CaptureAware(dev)
 
 
 def _native(name, *args):

@@ -70,6 +70,6 @@ def test_missing_library_leaves_the_device(monkeypatch):
 
     monkeypatch.setattr(_ffi, "load", missing)
     with pytest.raises(OSError, match="no library"):
-        with op._on(torch.device("cuda", 0)):
+        with op._CaptureAware(torch.device("cuda", 0)):
             pass
     assert not entered
